@@ -62,6 +62,43 @@ def test_prefill_router_kernelcheck(tsg, ctx, t, kind, seed):
     assert worst <= kc.FP16_REDUCTION
 
 
+@pytest.mark.parametrize("t,ne,d", [
+    (9, 128, 2816), (16, 13, 8), (17, 8, 520), (33, 96, 768), (65, 128, 1544), (301, 256, 2048),
+    (31, 130, 2568), (47, 129, 3584), (40, 256, 4096), (2048, 128, 2816), (2049, 127, 3072),
+])
+def test_prompt_router_equals_decode_router(tsg, ctx, t, ne, d):
+    """The prompt router's ids and weights equal the one-row decode router's
+    bit for bit, at row and expert counts around its tiles and at d with a full
+    and a partial last chunk. Experts 1 and ne - 1 share a row (exact ties);
+    row 3 is zero (every logit ties), row 4 is NaN (nothing is eligible). The
+    rows are strided."""
+    configure(ctx, 32, "sym")
+    rng = np.random.default_rng(t + ne + d)
+    stride = d + 8
+    hidden = rng.normal(size=(t, stride)).astype(np.float16)
+    hidden[3] = 0.0
+    hidden[4] = np.nan
+    w = rng.normal(0.0, d ** -0.5, (ne, d)).astype(np.float32)
+    w[ne - 1] = w[1]
+    W, X = dev(oracle.bf16_bits(w).ravel()), dev(hidden.view(np.uint16).ravel())
+    es = dev(oracle.bf16_bits(rng.uniform(0.5, 1.5, d).astype(np.float32)))
+    pes = dev(oracle.bf16_bits(rng.uniform(0.5, 1.5, ne).astype(np.float32)))
+    moe = tsg.MoE(ctx)
+    idx, wts = empty(t * 8, np.uint32), empty(t * 8)
+    for _ in range(2):  # the second call finds the row counters as the first left them
+        idx.fill_(-1), wts.fill_(-1)
+        tsg.PrefillRouter(moe).encode_gemma4_bf16(W, X, stride, es, pes, idx, wts, t, ne, d)
+    gi = host(idx, np.uint32).reshape(t, 8)
+    gw = host(wts, np.uint16).reshape(t, 8)
+    rows = sorted({*range(min(t, 20)), t // 2, t - 17 if t > 17 else 0, t - 2, t - 1})
+    one_i, one_w = empty(len(rows) * 8, np.uint32), empty(len(rows) * 8)
+    for q, row in enumerate(rows):
+        moe.encode_router_gemma4_bf16(W, X[row * stride:row * stride + d], es, pes,
+                                      one_i[8 * q:8 * q + 8], one_w[8 * q:8 * q + 8], ne, d)
+    assert np.array_equal(gi[rows], host(one_i, np.uint32).reshape(-1, 8))
+    assert np.array_equal(gw[rows], host(one_w, np.uint16).reshape(-1, 8))
+
+
 def _upload_layer(tsg, ctx, expert_parts, symmetric):
     image, stride, offs, blobs = kc.layer_image(expert_parts, symmetric, keep_biases=not symmetric)
     layer = tsg.ResidentLayer(ctx, len(expert_parts), stride, offs)

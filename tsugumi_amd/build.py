@@ -22,7 +22,8 @@ FLOORS_LIB = os.path.join(HERE, "libtsugumi_floors.so")
 # scheme), in parallel with the rest
 GEMM_SOURCES = ["gemm_g32_sym.hip", "gemm_g32_affine.hip", "gemm_g64_sym.hip",
                 "gemm_g64_affine.hip"]
-SOURCES = ["core.hip", "decode.hip", "qmv.hip", "shared.hip", "prefill.hip", "tail.hip",
+SOURCES = ["core.hip", "decode.hip", "prompt_router.hip", "qmv.hip", "shared.hip", "prefill.hip",
+           "tail.hip",
            *GEMM_SOURCES,
            "host_routing.cpp",
            "moepack.cpp"]

@@ -8,7 +8,7 @@
 //    c = l, l+64, ... in order with fma, then a xor butterfly over the 64
 //    lanes (32, 16, 8, 4, 2, 1). The oracle restates exactly this order, which is
 //    what makes the selected experts bit-exact (and identical between decode
-//    and the prompt router, which runs the same body per row).
+//    and the prompt router, prompt_router.hip, which keeps the order).
 //  * phase 1: 8 lanes own one (slot, f) row pair of gate and up. Lane j streams
 //    16-byte chunks j, j+8, ... (one g32 group each) with all of its loads in
 //    flight at once, converts nibbles to fp16 with the 0x6400 exponent trick
@@ -18,6 +18,7 @@
 //    values of a row are combined in slot order in one lane, as the reference
 //    does (moe.metal:678-686).
 #include "qwen_shared.hpp"
+#include "router_select.hpp"
 
 namespace tsg {
 namespace {
@@ -62,8 +63,7 @@ struct LdsBlobs {
 // per-expert gain, rounded to fp16. Runs on one full wave; lane l holds the
 // logits of experts l + 64 j (j < 4). Every lane returns the same result.
 //
-// Scores become order-preserving 32-bit keys (0 marks "not eligible"; -0 is
-// keyed as +0, the two compare equal). Each round takes the wave-wide max key
+// Scores become order_key's 32-bit keys. Each round takes the wave-wide max key
 // on DPP moves inside 16-lane rows and permlane swaps across rows, then the
 // lowest expert holding it from per-j ballots (experts l + 64 j ascend with j
 // and, within j, with the lane).
@@ -71,20 +71,6 @@ struct TopK {
     uint32_t idx[kTopK];
     uint16_t w[kTopK];
 };
-
-__device__ __forceinline__ uint32_t order_key(float v) {
-    const uint32_t u = __float_as_uint(v + 0.0f);  // -0 -> +0
-    return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-}
-
-__device__ __forceinline__ float order_key_value(uint32_t k) {
-    return __uint_as_float((k & 0x80000000u) ? (k & 0x7FFFFFFFu) : ~k);
-}
-
-template <int CTRL>
-__device__ __forceinline__ uint32_t dpp_u32(uint32_t k) {
-    return __builtin_amdgcn_update_dpp(0u, k, CTRL, 0xF, 0xF, false);
-}
 
 // Of the two results of a permlane swap each lane finds its partner's value
 // in one and its own in the other, so the max of both is the pairwise max
@@ -201,7 +187,6 @@ __device__ void wave_topk_softmax(const float* logits, uint32_t ne, const uint32
     }
 }
 
-constexpr uint32_t kRouterRows = 16;      // rows sharing one weight read per wave
 constexpr uint32_t kRouterWaves = 4;      // experts per block
 constexpr int kRouterChunks = 8;          // 8-element chunks per lane: d <= 4096
 
@@ -843,17 +828,16 @@ __device__ void group_router_rows(const uint32_t* pe, const uint32_t* pw, uint32
     if (t == 0) g.n_blocks[0] = total >> 16;
 }
 
-// One expert row against up to kRouterRows activation rows in the canonical
+// One expert row against up to kMaxRouterRows activation rows in the canonical
 // order: lane l sums chunks l, l+64, ... (elements in order, acc = fma(w,
 // x*es, acc)); each 16-lane row then sums as group16_sum does (pairs, pairs of
 // pairs, mirrored quads, mirrored 8s) and the four row sums add as
 // (r0 + r1) + (r2 + r3). Every lane ends with the full sum. Loads for all
 // chunks are issued before any arithmetic; out-of-range chunks load a clamped
 // address and contribute nothing.
-//  - one row or a prompt's rows: block b holds experts 4b .. 4b + 3, one per
-//    wave, each wave taking the rows in turn (the next row's activations
-//    requested before this row's sums); the last block ranks each row on one
-//    wave (wave_topk_softmax).
+//  - one row: block b holds experts 4b .. 4b + 3, one per wave; the last block
+//    ranks the row on one wave (wave_topk_softmax). More rows than the staged
+//    form takes go to the prompt router (prompt_router.hip).
 //  - STAGE (2..8 rows, or GROUP): block e holds expert e and copies the rows
 //    to LDS once, after its weight row is requested; wave w takes rows w,
 //    w + 4. The last block ranks each row on one wave with the candidate
@@ -872,16 +856,14 @@ __global__ __launch_bounds__(STAGE ? 64u * kStageWaves : 256u) void router_kerne
     const uint16_t* __restrict__ w, const uint16_t* __restrict__ hidden,
     const uint16_t* __restrict__ es, const uint16_t* __restrict__ pes,
     uint32_t* __restrict__ counters, uint32_t hidden_stride, uint32_t ne, uint32_t d,
-    uint32_t rows, float* __restrict__ logits, uint32_t logits_stride,
-    uint32_t* __restrict__ out_idx, uint16_t* __restrict__ out_w, uint32_t top_k,
+    uint32_t rows, float* __restrict__ logits, uint32_t* __restrict__ out_idx, uint16_t* __restrict__ out_w, uint32_t top_k,
     RouterGroupOut grp) {
     static_assert(!GROUP || (SELECT && STAGE), "the grouping follows a staged selection");
     static_assert(!STAGE || SELECT, "the staged form selects");
     extern __shared__ __align__(16) uint4 xrows[];  // STAGE: the block's rows, d / 8 units each
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint32_t e = STAGE ? blockIdx.x : blockIdx.x * kRouterWaves + wave;
-    const uint32_t r0 = blockIdx.y * kRouterRows;
-    const uint32_t nr = min(kRouterRows, rows - r0);
+    const uint32_t nr = STAGE ? rows : 1u;
     const uint32_t nchunks = d / 8u;
     uint32_t gains[4] = {0u, 0u, 0u, 0u};
     if constexpr (SELECT && !STAGE) load_expert_gains(pes, ne, gains);
@@ -904,7 +886,7 @@ __global__ __launch_bounds__(STAGE ? 64u * kStageWaves : 256u) void router_kerne
             wv[i] = *reinterpret_cast<const uint4*>(wr + cc * 8u);
             ev[i] = *reinterpret_cast<const uint4*>(es + cc * 8u);
             if constexpr (!STAGE)
-                xv[i] = *reinterpret_cast<const uint4*>(hidden + (uint64_t)r0 * hidden_stride + cc * 8u);
+                xv[i] = *reinterpret_cast<const uint4*>(hidden + cc * 8u);
         }
     }
     __shared__ uint32_t s_tag;
@@ -921,7 +903,7 @@ __global__ __launch_bounds__(STAGE ? 64u * kStageWaves : 256u) void router_kerne
             for (uint32_t i = 0; i < kStageUnits; ++i) {
                 const uint32_t q = min(q0 + threadIdx.x + i * blockDim.x, total - 1u);
                 const uint32_t r = q / nchunks, c = q - r * nchunks;
-                v[i] = *reinterpret_cast<const u32x4_t*>(hidden + (uint64_t)(r0 + r) * hidden_stride + c * 8u);
+                v[i] = *reinterpret_cast<const u32x4_t*>(hidden + (uint64_t)r * hidden_stride + c * 8u);
             }
             // keeps the compiler from sinking each load into its conditional
             // store below (which would make the round trips serial again)
@@ -945,23 +927,9 @@ __global__ __launch_bounds__(STAGE ? 64u * kStageWaves : 256u) void router_kerne
                 st_coherent(r_logits + (uint64_t)r * kMaxExperts + e, tagged(tag, __float_as_uint(acc)));
         }
     } else if (e < ne) {
-        for (uint32_t r = 0; r < nr; ++r) {
-            // next row's activations go out before this row's arithmetic
-            uint4 xn[kRouterChunks];
-            const uint32_t rn = (r + 1 < nr) ? r + 1 : r;
-            const uint16_t* xnext = hidden + (uint64_t)(r0 + rn) * hidden_stride;
-#pragma unroll
-            for (int i = 0; i < kRouterChunks; ++i) {
-                const uint32_t cc = min(lane + 64u * i, nchunks - 1u);
-                xn[i] = *reinterpret_cast<const uint4*>(xnext + cc * 8u);
-            }
-            const float acc = router_chunks_dot(wv, xv, ev, nchunks, lane);
-#pragma unroll
-            for (int i = 0; i < kRouterChunks; ++i) xv[i] = xn[i];
-            if (lane == 0)
-                st_coherent(reinterpret_cast<uint32_t*>(logits) + (uint64_t)(r0 + r) * logits_stride + e,
-                            __float_as_uint(acc));
-        }
+        const float acc = router_chunks_dot(wv, xv, ev, nchunks, lane);
+        if (lane == 0)
+            st_coherent(reinterpret_cast<uint32_t*>(logits) + e, __float_as_uint(acc));
     }
     if constexpr (SELECT) {
         // STAGE: block 0 selects, polling the other blocks' tagged logits (the
@@ -977,7 +945,7 @@ __global__ __launch_bounds__(STAGE ? 64u * kStageWaves : 256u) void router_kerne
             wait_vector_memory();
             __syncthreads();
             if (threadIdx.x == 0) {
-                const uint32_t done = atomicAdd(&counters[blockIdx.y], 1u);
+                const uint32_t done = atomicAdd(&counters[0], 1u);
                 is_last = (done == gridDim.x - 1u) ? 1u : 0u;
             }
             __syncthreads();
@@ -1038,18 +1006,15 @@ __global__ __launch_bounds__(STAGE ? 64u * kStageWaves : 256u) void router_kerne
                     group_router_rows(s_pe, s_pw, nr * kTopK, ne, gl, grp);
                 }
                 if (my_pair) {
-                    out_idx[(uint64_t)r0 * kTopK + t] = my_id;
-                    out_w[(uint64_t)r0 * kTopK + t] = (uint16_t)my_wb;
+                    out_idx[t] = my_id;
+                    out_w[t] = (uint16_t)my_wb;
                 }
                 // every block has posted (the polls saw all tags): the next
                 // launch may use tag + 1
                 if (t == 0) st_coherent(r_epoch, s_tag);
             } else {
-                for (uint32_t r = wave; r < nr; r += kRouterWaves)
-                    wave_topk_softmax(logits + (uint64_t)(r0 + r) * logits_stride, ne, gains,
-                                      out_idx + (uint64_t)(r0 + r) * kTopK,
-                                      out_w + (uint64_t)(r0 + r) * kTopK);
-                if (threadIdx.x == 0) atomicExch(&counters[blockIdx.y], 0u);
+                if (wave == 0) wave_topk_softmax(logits, ne, gains, out_idx, out_w);
+                if (threadIdx.x == 0) atomicExch(&counters[0], 0u);
             }
         }
     }
@@ -2243,12 +2208,13 @@ tsg_status router_launch(tsg_moe* moe, hipStream_t stream, const uint16_t* w,
     TSG_REQUIRE(moe->router_weight_bits == 16, TSG_ERR_INVALID_ARGUMENT,
                 "BF16 router encode on a %u-bit router", moe->router_weight_bits);
     tsg_ctx* ctx = moe->ctx;
-    const dim3 grid((ne + kRouterWaves - 1) / kRouterWaves, (rows + kRouterRows - 1) / kRouterRows);
-    // a few rows of one y-block are staged in LDS (same sums, no per-row
-    // round trip to memory); the one-row and prompt-sized forms are not
+    const dim3 grid((ne + kRouterWaves - 1) / kRouterWaves);
+    // a few rows are staged in LDS (same sums, no per-row round trip to
+    // memory); more take the prompt router
     const size_t stage = (size_t)rows * d * 2u;
     const bool staged = select && (rows > 1 || group) && rows <= kMaxRouterRows &&
                         stage <= 64u * 1024u;
+    TSG_REQUIRE(select || rows == 1, TSG_ERR_INVALID_ARGUMENT, "logits of one row only, got %u", rows);
     TSG_REQUIRE(!group || staged, TSG_ERR_UNSUPPORTED,
                 "the grouped router takes 1..%u rows of at most %zu bytes", kMaxRouterRows,
                 (size_t)64u * 1024u);
@@ -2257,6 +2223,9 @@ tsg_status router_launch(tsg_moe* moe, hipStream_t stream, const uint16_t* w,
         TSG_REQUIRE(top_k == kTopK, TSG_ERR_INVALID_ARGUMENT, "topK must be %u, got %u", kTopK,
                     top_k);
         TSG_REQUIRE(pes && out_idx && out_w, TSG_ERR_INVALID_ARGUMENT, "NULL router output");
+        if (rows > kMaxRouterRows)
+            return prompt_router_launch(ctx, stream, PromptRouterArgs{w, hidden, es, pes, out_idx,
+                                                                      out_w, stride, ne, d, rows});
         if (staged) {
             auto kern = group ? router_kernel<true, true, true> : router_kernel<true, true, false>;
             // the staged rows take up to 64 KiB of dynamic LDS (idempotent)
@@ -2265,17 +2234,16 @@ tsg_status router_launch(tsg_moe* moe, hipStream_t stream, const uint16_t* w,
                                             64 * 1024));
             hipLaunchKernelGGL(kern, sgrid, dim3(64u * kStageWaves), stage, stream, w, hidden,
                                es, pes, ctx->counters, stride, ne, d, rows, ctx->logits,
-                               kMaxExperts, out_idx, out_w, top_k,
-                               group ? *group : RouterGroupOut{});
+                               out_idx, out_w, top_k, group ? *group : RouterGroupOut{});
         }
         else
             hipLaunchKernelGGL((router_kernel<true, false, false>), grid, dim3(256), 0, stream, w,
                                hidden, es, pes, ctx->counters, stride, ne, d, rows, ctx->logits,
-                               kMaxExperts, out_idx, out_w, top_k, RouterGroupOut{});
+                               out_idx, out_w, top_k, RouterGroupOut{});
     } else {
         TSG_REQUIRE(logits_out, TSG_ERR_INVALID_ARGUMENT, "out_logits is NULL");
         hipLaunchKernelGGL((router_kernel<false, false, false>), grid, dim3(256), 0, stream, w,
-                           hidden, es, pes, ctx->counters, stride, ne, d, rows, logits_out, ne,
+                           hidden, es, pes, ctx->counters, stride, ne, d, rows, logits_out,
                            out_idx, out_w, top_k, RouterGroupOut{});
     }
     return check_launch("router");
@@ -2808,8 +2776,7 @@ extern "C" tsg_status tsg_moe_set_fused_decode(tsg_moe* moe, int enabled) {
     return TSG_OK;
 }
 
-// Prompt router: the decode router body per row (bit-identical per row), all
-// rows in one launch.
+// Prompt router: the decode router's result per row, bit for bit.
 extern "C" tsg_status tsg_prefill_router_bf16(tsg_moe* moe, tsg_stream stream,
                                               const uint16_t* w, const uint16_t* hidden,
                                               uint32_t stride, const uint16_t* es,
