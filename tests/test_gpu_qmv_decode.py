@@ -7,6 +7,7 @@ import pytest
 
 import oracle
 from tests import kernelcheck as kc
+from tests import workloads as wl
 from tests.gpu_util import dev, empty, host
 
 pytestmark = pytest.mark.gpu
@@ -631,6 +632,39 @@ def test_decode_layer_shared_expert(tsg, ctx, d, f, ne, sf, group, scheme):
     rel = oracle.relative_error(oracle.f16_to_float(y), ref)
     print(f"  rel={rel:.3e}")
     assert rel <= kc.NORTH_STAR
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n", [(1, 64), (17, 3072), (33, 3136), (48, 4096), (15, 4160), (31, 8256)])
+@pytest.mark.parametrize("group,scheme", [(32, "sym"), (64, "affine")])
+def test_qmv_row_lengths_around_the_batches(tsg, ctx, m, n, group, scheme):
+    """One batch of six chunks a lane covers n = 3072, one of eight n = 4096;
+    beyond, batches follow each other. Every row count gives the one-row
+    result bit for bit, and that is DequantInt4GemvRef's within 1e-3."""
+    configure(ctx, group, scheme)
+    sym = scheme == "sym"
+    rng = np.random.default_rng(m + n)
+    w = rng.integers(0, 256, m * n // 2, dtype=np.uint8)
+    s = wl.scale_bits(rng, m * n // group)
+    b = None if sym else oracle.bf16_bits(-7.5 * oracle.bf16_to_float(s))
+    xs = wl.f16_normal(rng, 8 * n)
+    W, S, X = dev(w), dev(s), dev(xs)
+    B = S if sym else dev(b)
+    gemv = tsg.DequantInt4GEMV(ctx)
+    one = empty(8 * m)
+    for r in range(8):
+        gemv.encode(W, S, B, X[r * n:(r + 1) * n], one[r * m:(r + 1) * m], m, n)
+    want = host(one, np.uint16).reshape(8, m)
+    for t in range(1, 9):
+        y = empty(t * m)
+        gemv.encode_rows(W, S, B, X, n, y, m, t, m, n)
+        assert np.array_equal(host(y, np.uint16).reshape(t, m), want[:t]), t
+    q = np.stack([w & 15, w >> 4], axis=-1).reshape(m, n).astype(np.float64)
+    scale = np.repeat(oracle.bf16_to_float(s).reshape(m, -1), group, axis=1).astype(np.float64)
+    bias = -8.0 * scale if sym else np.repeat(
+        oracle.bf16_to_float(b).reshape(m, -1), group, axis=1).astype(np.float64)
+    ref = (q * scale + bias) @ oracle.f16_to_float(xs).reshape(8, n).astype(np.float64).T
+    assert oracle.relative_error(oracle.f16_to_float(want.ravel()), ref.T.ravel()) <= kc.NORTH_STAR
 
 
 @pytest.mark.gpu

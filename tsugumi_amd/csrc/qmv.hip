@@ -6,6 +6,14 @@
 // exponent trick, v_dot2_f32_f16 against x staged in LDS, fp32 scale fma.
 // The rows form keeps T <= 8 accumulators per lane so a weight chunk is read
 // once for all rows; each row's sum runs in exactly the one-row order.
+//
+// What bounds it: latency (a launch is 2-2.5 us, the rest the round trip of
+// staging and weights and, for several rows, a lane's dot2 chains and LDS
+// reads at one wave a SIMD). Back to back in a HIP graph over weights that no
+// cache holds, us before and now, group 32 sym: 704 x 2816 3.90 -> 3.26, 2816 x
+// 4096 6.12 -> 4.23, 4096 x 2816 3.95 -> 3.82; five rows of them 9.25 -> 5.98,
+// 15.95 -> 7.75, 7.23 -> 6.42; group 64 affine 2816 x 4096 6.35 -> 4.86, five
+// rows 17.5 -> 10.2, eight 68 -> 14.3.
 #include "gemv_lane.hpp"
 
 namespace tsg {
@@ -13,26 +21,73 @@ namespace {
 
 constexpr uint32_t kMaxRows = 8;
 
-// WA: the weights' alignment, 16 or 2 (a weights pointer bound at a 2-byte
-// offset, DequantInt4GEMV.swift:93-96: every row starts at the same offset
-// modulo 16, since a row is a multiple of 16 bytes).
-// RPB rows per block (16 lanes each), so the block size is a constant. The
-// parameters the first loads need fill the first 14 dwords, which the
+// compute_batch for T token rows, the rows' dot2 chains side by side (one
+// after the other, a wave waits for each dot2 of a 16-long chain: eight rows of
+// 8192 x 2816 12.1 us against 10.9, of 2816 x 4096 14.7 against 10.4). Each row takes compute_batch's steps.
+template <int G, bool SYM, int KB, int T>
+__device__ __forceinline__ void compute_rows(const ChunkBatch<KB>& bt, uint32_t base, uint32_t j,
+                                             uint32_t nchunks, const uint16_t* xs, uint32_t row_h,
+                                             const float* xsum, float (&acc)[T]) {
+    const h2_t bias = SYM ? h2_t{(_Float16)1032.0f, (_Float16)1032.0f}
+                          : h2_t{(_Float16)1024.0f, (_Float16)1024.0f};
+#pragma unroll
+    for (int i = 0; i < KB; ++i) {
+        const uint32_t c = base + j + kGULanes * i;
+        const uint32_t cc = min(c, nchunks - 1u);
+        const uint32_t w[4] = {bt.w[i].x, bt.w[i].y, bt.w[i].z, bt.w[i].w};
+        float dot[T];
+#pragma unroll
+        for (int r = 0; r < T; ++r) dot[r] = 0.0f;
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            h2_t q[4];
+            nib8_to_pairs(w[b], bias, q);
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+#pragma unroll
+                for (int r = 0; r < T; ++r)
+                    dot[r] = dot2(q[k], staged_chunk(xs + (size_t)r * row_h, cc)[4 * b + k], dot[r]);
+        }
+        const float s = bf16_to_f32((uint16_t)bt.s[i]);
+        float bi = 0.0f;
+        if constexpr (!SYM) bi = bf16_to_f32((uint16_t)bt.b[i]);
+#pragma unroll
+        for (int r = 0; r < T; ++r) {
+            float v = __builtin_fmaf(s, dot[r], acc[r]);
+            if constexpr (!SYM) v = __builtin_fmaf(bi, xsum[r * nchunks + cc], v);
+            acc[r] = c < nchunks ? v : acc[r];  // a chunk past the row end leaves acc as it is
+        }
+    }
+}
+
+constexpr uint32_t kRowsPerBlock = 16;  // weight rows a block, 16 lanes each
+constexpr uint32_t kQmvThreads = 16u * kRowsPerBlock;
+constexpr int kOneBatch = 6;  // chunks a lane loads when they are the whole row (n <= 3072)
+
+// T token rows. WA: the weights' alignment, 16 or 2 (a weights pointer bound
+// at a 2-byte offset, DequantInt4GEMV.swift:93-96: every row starts at the
+// same offset modulo 16, since a row is a multiple of 16 bytes). KB: chunks a
+// lane loads at once: kOneBatch, or 8 with the batch after requested before
+// this one's sums.
+// The parameters the first loads need fill the first 14 dwords, which the
 // dispatch preloads into SGPRs: no kernel-argument load comes before them.
-template <int G, bool SYM, int T, int WA, uint32_t RPB>
-__global__ __launch_bounds__(16 * RPB) void qmv_kernel(const uint8_t* __restrict__ w,
-                                                       const uint16_t* __restrict__ scales,
-                                                       const uint16_t* __restrict__ biases,
-                                                       const uint16_t* __restrict__ x,
-                                                       uint16_t* __restrict__ y, uint32_t n,
-                                                       uint32_t m, uint32_t t, uint32_t x_stride,
-                                                       uint32_t y_stride) {
+// Every block stages the token rows: with 4 weight rows a block (one wave) the
+// staging took up to ten round trips to memory, and its LDS left three waves
+// to a compute unit (five rows of 2816 x 4096: 15.7 us against 11.4 with 16).
+template <int G, bool SYM, int T, int WA, int KB>
+__global__ __launch_bounds__(kQmvThreads) void qmv_kernel(const uint8_t* __restrict__ w,
+                                                          const uint16_t* __restrict__ scales,
+                                                          const uint16_t* __restrict__ biases,
+                                                          const uint16_t* __restrict__ x,
+                                                          uint16_t* __restrict__ y, uint32_t n,
+                                                          uint32_t m, uint32_t x_stride,
+                                                          uint32_t y_stride) {
     extern __shared__ __align__(16) uint8_t smem[];
     const uint32_t row_h = lds_chunks_halves(n);
     uint16_t* xs = reinterpret_cast<uint16_t*>(smem);                        // T rows
     float* xsum = reinterpret_cast<float*>(smem + (size_t)T * row_h * 2u);  // T * n / 32
 
-    const uint32_t row = blockIdx.x * RPB + (threadIdx.x >> 4);
+    const uint32_t row = blockIdx.x * kRowsPerBlock + (threadIdx.x >> 4);
     const uint32_t j = threadIdx.x & 15u;
     const bool live = row < m;
     const uint32_t rr = live ? row : 0u;
@@ -40,25 +95,33 @@ __global__ __launch_bounds__(16 * RPB) void qmv_kernel(const uint8_t* __restrict
     const uint8_t* wr = w + (uint64_t)rr * (n / 2u);
     const uint16_t* sr = scales + (uint64_t)rr * ngroups;
     const uint16_t* br = biases + (uint64_t)rr * ngroups;
-    ChunkBatch<kGUBatch> bt;
-    auto issue_weights = [&] {
-        load_batch<G, SYM, kGUBatch, kGULanes, WA>(wr, sr, br, 0u, j, nchunks, bt);
-    };
-    stage_act_rows_around<SYM, decltype(issue_weights)&, 4, 16u * RPB>(x, x_stride, t, n, xs, row_h,
-                                                                       xsum, nullptr, issue_weights);
+    ChunkBatch<KB> bt;
+    auto issue_weights = [&] { load_batch<G, SYM, KB, kGULanes, WA>(wr, sr, br, 0u, j, nchunks, bt); };
+    constexpr int kPer = T == 1 ? 4 : T <= 4 ? 8 : 12;
+    stage_act_rows_around<SYM, decltype(issue_weights)&, kPer, kQmvThreads>(
+        x, x_stride, T, n, xs, row_h, xsum, nullptr, issue_weights);
     __syncthreads();
     float acc[T];
 #pragma unroll
     for (int r = 0; r < T; ++r) acc[r] = 0.0f;
-    gemv_batches<G, SYM, kGUBatch, kGULanes, T, WA>(wr, sr, br, j, nchunks, bt, xs, row_h, xsum, t, acc);
+    uint32_t base = 0u;
+    if constexpr (KB > kOneBatch) {
+        constexpr uint32_t kStep = kGULanes * KB;
+        for (; base + kStep < nchunks; base += kStep) {
+            ChunkBatch<KB> next;
+            load_batch<G, SYM, KB, kGULanes, WA>(wr, sr, br, base + kStep, j, nchunks, next);
+            compute_rows<G, SYM, KB, T>(bt, base, j, nchunks, xs, row_h, xsum, acc);
+            bt = next;
+        }
+    }
+    compute_rows<G, SYM, KB, T>(bt, base, j, nchunks, xs, row_h, xsum, acc);
 #pragma unroll
     for (int r = 0; r < T; ++r) {
         acc[r] = group16_sum(acc[r]);
     }
     if (live && j == 0) {
 #pragma unroll
-        for (int r = 0; r < T; ++r)
-            if ((uint32_t)r < t) y[(uint64_t)r * y_stride + row] = f32_to_f16(acc[r]);
+        for (int r = 0; r < T; ++r) y[(uint64_t)r * y_stride + row] = f32_to_f16(acc[r]);
     }
 }
 
@@ -88,20 +151,15 @@ template <int G, bool SYM, int WA>
 tsg_status launch_qmv(hipStream_t s, const uint8_t* w, const uint16_t* sc, const uint16_t* bi,
                       const uint16_t* x, uint32_t xs, uint16_t* y, uint32_t ys, uint32_t t,
                       uint32_t m, uint32_t n) {
-    // 16 lanes per row; 4 rows per block (one wave) below 4096 rows so a
-    // small matrix still spreads over the CUs, 16 above
-    const uint32_t rpb = m < 4096u ? 4u : 16u;
-    const dim3 grid((m + rpb - 1u) / rpb), block(16u * rpb);
-    const size_t lds_per_row = (size_t)lds_chunks_halves(n) * 2u + (SYM ? 0u : (n / 32u) * 4u);
-#define TSG_QMV_CASE(TT)                                                                        \
-    case TT:                                                                                    \
-        if (rpb == 4u)                                                                          \
-            hipLaunchKernelGGL((qmv_kernel<G, SYM, TT, WA, 4u>), grid, block, lds_per_row * TT, \
-                               s, w, sc, bi, x, y, n, m, t, xs, ys);                            \
-        else                                                                                    \
-            hipLaunchKernelGGL((qmv_kernel<G, SYM, TT, WA, 16u>), grid, block, lds_per_row * TT, \
-                               s, w, sc, bi, x, y, n, m, t, xs, ys);                            \
-        break;
+    const dim3 grid((m + kRowsPerBlock - 1u) / kRowsPerBlock), block(kQmvThreads);
+    const size_t lds = (size_t)t * (lds_chunks_halves(n) * 2u + (SYM ? 0u : (n / 32u) * 4u));
+    const bool one = n <= 32u * kGULanes * (uint32_t)kOneBatch;
+#define TSG_QMV_CASE(TT)                                                                          \
+    case TT: {                                                                                    \
+        auto kern = one ? qmv_kernel<G, SYM, TT, WA, kOneBatch> : qmv_kernel<G, SYM, TT, WA, 8>;  \
+        hipLaunchKernelGGL(kern, grid, block, lds, s, w, sc, bi, x, y, n, m, xs, ys);             \
+        break;                                                                                    \
+    }
     switch (t) {
         TSG_QMV_CASE(1)
         TSG_QMV_CASE(2)

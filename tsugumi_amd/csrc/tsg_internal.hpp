@@ -398,17 +398,26 @@ __device__ __forceinline__ uint4 pair_permute(uint4 v) {
 }
 
 // The fp32 sum of each 32-element chunk of `rows` staged rows, in element
-// order, into sums[r * n/32 + c] (the affine scheme's bias term). The staged
-// rows must be visible to the block (the caller synchronises before).
+// order, into sums[r * n/32 + c] (the affine scheme's bias term), from four
+// 16-byte reads a chunk. The staged rows must be visible to the block (the caller synchronises before).
 __device__ __forceinline__ void staged_chunk_sums(const uint16_t* dst, uint32_t dst_stride,
                                                   uint32_t rows, uint32_t n, float* sums) {
     const uint32_t cpr = n / 32u;
     for (uint32_t q = threadIdx.x; q < rows * cpr; q += blockDim.x) {
         const uint32_t r = q / cpr, c = q - r * cpr;
-        const uint16_t* chunk = dst + (size_t)r * dst_stride + c * kChunkLds;
+        const uint4* chunk = reinterpret_cast<const uint4*>(dst + (size_t)r * dst_stride + c * kChunkLds);
+        uint4 v[4];
+#pragma unroll
+        for (int b = 0; b < 4; ++b) v[b] = chunk[b];
         float s = 0.0f;
-        for (uint32_t k = 0; k < 32u; ++k)
-            s += f16_to_f32(chunk[(k >> 3) * 8u + paired_pos(k & 7u)]);
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            const uint32_t u[4] = {v[b].x, v[b].y, v[b].z, v[b].w};  // (e0,e4) (e1,e5) (e2,e6) (e3,e7)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) s += f16_to_f32((uint16_t)(u[k] & 0xFFFFu));
+#pragma unroll
+            for (int k = 0; k < 4; ++k) s += f16_to_f32((uint16_t)(u[k] >> 16));
+        }
         sums[q] = s;
     }
 }
