@@ -634,6 +634,32 @@ def test_decode_layer_shared_expert(tsg, ctx, d, f, ne, sf, group, scheme):
     assert rel <= kc.NORTH_STAR
 
 
+def test_default_stream_is_torchs_current_stream(tsg, ctx):
+    """Calls without a stream go to torch's current stream, inside a stream
+    context and out of it, in this thread and in another."""
+    import threading
+
+    import torch
+    side, other = torch.cuda.Stream(), torch.cuda.Stream()
+    assert tsg._stream(None) == torch.cuda.current_stream().cuda_stream
+    with torch.cuda.stream(side):
+        assert tsg._stream(None) == side.cuda_stream
+        seen = []
+
+        def work():
+            seen.append(tsg._stream(None) == torch.cuda.current_stream().cuda_stream)
+            with torch.cuda.stream(other):
+                seen.append(tsg._stream(None) == other.cuda_stream)
+
+        th = threading.Thread(target=work)
+        th.start()
+        th.join()
+        assert seen == [True, True]
+        assert tsg._stream(None) == side.cuda_stream
+    assert tsg._stream(None) == torch.cuda.current_stream().cuda_stream
+    assert tsg._stream(other) == other.cuda_stream and tsg._stream(5) == 5
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,n", [(1, 64), (17, 3072), (33, 3136), (48, 4096), (15, 4160), (31, 8256)])
 @pytest.mark.parametrize("group,scheme", [(32, "sym"), (64, "affine")])

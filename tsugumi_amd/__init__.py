@@ -58,11 +58,34 @@ def _ptr(t) -> int | None:
     return t.data_ptr()
 
 
+def _stream_reader():
+    """A function that returns torch's current stream on the current device as
+    an address. Once torch has initialised the device it reads the address
+    itself (0.3 us a call on the host): torch.cuda.current_stream() builds a
+    Stream object around it (2.9 us, a third of a small call)."""
+    import torch
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    device = getattr(torch._C, "_cuda_getDevice", None)
+    initialised = torch.cuda.is_initialized
+
+    def read() -> int:
+        if raw is not None and device is not None and initialised():
+            return raw(device())
+        return torch.cuda.current_stream().cuda_stream
+
+    return read
+
+
+_current_stream = None
+
+
 def _stream(stream) -> int | None:
     if stream is not None:
         return stream if isinstance(stream, int) else stream.cuda_stream
-    import torch
-    return torch.cuda.current_stream().cuda_stream
+    global _current_stream
+    if _current_stream is None:
+        _current_stream = _stream_reader()
+    return _current_stream()
 
 
 def _np_ptr(a: np.ndarray):
