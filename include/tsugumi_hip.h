@@ -468,9 +468,9 @@ tsg_status tsg_gelu_mul_f16(tsg_ctx* ctx, tsg_stream stream, const uint16_t* gat
                             const uint16_t* up, uint16_t* out, uint32_t count);
 
 /* SharedExpertInt4.encode (Kernels/MoE/SharedExpertInt4.swift:30-93): Gemma's
- * dense int4 MLP, y = down(half(gelu(gate x) * up x)), as the reference
- * encodes it (QMV gate, QMV up, gelu_mul_fp16, QMV down), so the result is
- * bit-identical to those four calls. The byte lengths stand in for the
+ * dense int4 MLP, y = down(half(gelu(gate x) * up x)), bit-identical to the
+ * four calls the reference encodes (QMV gate, QMV up, gelu_mul_fp16, QMV
+ * down), in y and in the scratch. The byte lengths stand in for the
  * MTLBuffer lengths the reference checks: a mismatch of shapes returns
  * TSG_ERR_INVALID_ARGUMENT "dimensionMismatch: ...", a short buffer
  * "scratchTooSmall: ..." (SharedExpertError). */

@@ -193,6 +193,40 @@ def test_shared_expert_int4_matches_steps_and_oracle(tsg, ctx, d, f, group, symm
     assert rel <= kc.NORTH_STAR
 
 
+@pytest.mark.parametrize("d,f,group,symmetric", [(64, 64, 32, True), (3136, 64, 64, False),
+                                                 (128, 4160, 32, True), (4160, 992, 32, False)])
+def test_shared_expert_int4_scratch_and_shared_buffers(tsg, ctx, d, f, group, symmetric):
+    """At small and large f and at d past one batch of chunks: the scratch
+    holds the halves and the activation the separate calls leave there, and the
+    activation may share a buffer with a half or with x."""
+    configure(ctx, group, symmetric)
+    S, q = tsg.SharedExpertInt4(ctx), tsg.DequantInt4GEMV(ctx)
+    gate, up, down, x = _dense_parts(d, f, group, 0x71 + f, symmetric)
+    dv = [tuple(dev(a) for a in t) for t in (gate, up, down)]
+    bias = lambda t: t[1] if symmetric else t[2]
+    proj = [S.projection(t[0], t[1], bias(t), r, c)
+            for t, (r, c) in zip(dv, ((f, d), (f, d), (d, f)))]
+    g1, u1, a1, y1 = empty(f), empty(f), empty(f), empty(d)
+    q.encode(dv[0][0], dv[0][1], bias(dv[0]), dev(x), g1, f, d)
+    q.encode(dv[1][0], dv[1][1], bias(dv[1]), dev(x), u1, f, d)
+    S.encode_gelu_mul(g1, u1, a1, f)
+    q.encode(dv[2][0], dv[2][1], bias(dv[2]), a1, y1, d, f)
+    want = host(y1, np.uint16)
+    y, sg, su, sa = empty(d), empty(f), empty(f), empty(f)
+    S.encode(dev(x), *proj, y, sg, su, sa)
+    for got, ref in ((y, y1), (sg, g1), (su, u1), (sa, a1)):
+        assert np.array_equal(host(got, np.uint16), host(ref, np.uint16))
+    for g, u, a in ((sg, su, sg), (sg, su, su)):
+        y.fill_(0)
+        S.encode(dev(x), *proj, y, g, u, a)
+        assert np.array_equal(host(y, np.uint16), want)
+    both = empty(max(d, f))  # x and the activation in one buffer
+    both[:d] = dev(x)
+    y.fill_(0)
+    S.encode(both, *proj, y, sg, su, both)
+    assert np.array_equal(host(y, np.uint16), want)
+
+
 def test_shared_expert_int4_errors(tsg, ctx):
     """SharedExpertError.dimensionMismatch / .scratchTooSmall."""
     configure(ctx, 32, True)
