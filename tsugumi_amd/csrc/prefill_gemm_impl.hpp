@@ -684,7 +684,7 @@ __device__ __forceinline__ void gemm_block(const GemmArgs& args, const tsg_route
             }
         }
     }
-    block_barrier();
+    lds_barrier();  // the tile is written: block_barrier() waits for no LDS store
     const uint32_t col0 = MODE == 0 || HALF ? tile * 128u : tile * 256u;
     const uint32_t ncols = MODE == 0 ? args.f : args.d;
     const uint32_t live = ncols - col0 < kCols ? ncols - col0 : kCols;  // multiple of 64
