@@ -445,3 +445,48 @@ def test_gate_up_half_tile_equals_full_tile(tsg, ctx, group, scheme):
         out[f] = host(act, np.uint16).reshape(t * k, f)
     assert sorted(blocks["row_count"].tolist()) == [1, 31, 64, 96]
     assert np.array_equal(out[704], out[768][:, :704])
+
+
+@pytest.mark.parametrize("group,scheme,act", [(32, "sym", "silu"), (32, "affine", "gelu"),
+                                              (64, "sym", "gelu"), (64, "affine", "silu")])
+@pytest.mark.parametrize("d,f", [(512, 704), (320, 64), (64, 192), (832, 128)])
+def test_few_rows_gemms_equal_the_wide_ones(tsg, ctx, group, scheme, act, d, f):
+    """A device work list whose capacity is at most the experts + 6 runs the
+    three-per-CU kernels, one with spare capacity the wide ones: the same
+    activations and partials, bit for bit, from the one-launch entry and from
+    the two separate ones. Blocks of 1 to 200 rows: both slice counts, one to
+    four passes; K of 1 to 13 chunks (shorter than the ring, odd, ragged G = 64
+    windows); half and partial column tiles."""
+    sym = scheme == "sym"
+    configure(ctx, group, scheme)
+    rows = [1, 0, 31, 32, 33, 64, 65, 128, 129, 200]
+    ne, k = len(rows), 1
+    t = sum(rows)
+    rng = oracle.SplitMix64(0x7419)
+    parts = [[oracle.quantize_int4(rng.uniforms(-0.125, 0.125, r * c).reshape(r, c), group, sym)
+              for r, c in ((f, d), (f, d), (d, f))] for _ in range(ne)]
+    layer = _upload_layer(tsg, ctx, parts, sym)[0]
+    idx = np.repeat(np.arange(ne, dtype=np.uint32), rows).reshape(t, 1)
+    idx = idx[np.random.default_rng(3).permutation(t)]
+    w = np.full((t, k), 0x3800, np.uint16)
+    grouped = oracle.group_pairs(oracle.make_token_expert_pairs(idx, w, t, k), t, k, ne)
+    listed = wl.rows_blocks(grouped)  # one block per expert
+    hidden = dev(rng.uniforms_f16(-1, 1, t * d))
+    g = tsg.PrefillGroupedRoutedMoE(tsg.MoE(ctx, gate_activation=act))
+    P = dev(grouped["sorted_pairs"])
+    spare = ne + 40
+    B = dev(np.concatenate([listed, np.zeros(spare - listed.size, listed.dtype)]))
+    nb = dev(np.array([listed.size], np.uint32))
+    out = []
+    for cap, fused in ((spare, True), (spare, False), (ne + 6, True), (ne, False)):
+        a, p = empty(t * k * f, fill=NAN16), empty(t * k * d, fill=NAN16)
+        if fused:
+            g.encode_gate_up_down(layer, hidden, d, P, B, cap, a, p, k, d, f, n_blocks_device=nb)
+        else:
+            g.encode_gate_up(layer, hidden, d, P, B, cap, a, d, f, n_blocks_device=nb)
+            g.encode_down(layer, a, P, B, cap, p, k, d, f, n_blocks_device=nb)
+        out.append((host(a, np.uint16), host(p, np.uint16)))
+    ctx.synchronize()
+    assert not np.isnan(out[0][1].view(np.float16)).any()
+    for a, p in out[1:]:
+        assert np.array_equal(a, out[0][0]) and np.array_equal(p, out[0][1])

@@ -37,8 +37,8 @@ struct GemmArgs {
 
 // The routed GEMMs: mode 0 gate/up + activation, mode 1 down + scatter
 // (tsg_prefill_moe_gate_up / tsg_prefill_moe_down); both in one persistent
-// launch (tsg_prefill_moe_gate_up_down); the dense projection
-// (tsg_prefill_int4_qmm).
+// launch, or back to back for few rows an expert (tsg_prefill_moe_gate_up_down);
+// the dense projection (tsg_prefill_int4_qmm).
 template <int G, bool SYM>
 tsg_status routed_gemm_launch(const tsg_moe* moe, hipStream_t s, int mode, const GemmArgs& a,
                               uint32_t max_blocks);

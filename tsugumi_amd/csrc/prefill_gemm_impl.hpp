@@ -489,6 +489,106 @@ __device__ __forceinline__ void gemm_kloop(const GemmLane<NT>& L, uint8_t* smem,
     }
 }
 
+// ---- the K loop of the thin kernels (passes of at most kThinRows rows)
+//
+// A chunk's activations (NT slices), weights and one dword of group parameters
+// a row share an LDS stage; the loop over chunks is rolled, with the stage as
+// a run-time offset, kStages - 1 chunks ahead (3 of one slice, 2 of two). One
+// barrier a chunk: it publishes chunk c and frees chunk c - 1's stage. Every
+// accumulator sees gemm_kloop's MFMA sequence, so the results are the same.
+constexpr uint32_t kThinRows = 64u;
+constexpr uint32_t kThinLds = 53248u;  // three workgroups per CU
+template <bool SYM, int NT>
+struct ThinLds {
+    static constexpr uint32_t kB = NT * 4096u;                  // after the activations
+    static constexpr uint32_t kS = kB + kGemmBStage;            // 64 rows x 4 bytes a wave
+    static constexpr uint32_t kZ = kS + kGemmWaves * 256u;
+    static constexpr uint32_t kStage = kZ + (SYM ? 0u : kGemmWaves * 256u);
+    static constexpr uint32_t kStages = kThinLds / kStage;
+    static_assert(kStage % 128u == 0 && kStages >= 2u, "ring");
+};
+static_assert(GemmLds<kThinRows>::kEpi <= kThinLds && 3u * kThinLds <= 160u * 1024u, "three per CU");
+
+template <int G, bool SYM, int NT>
+__device__ __forceinline__ void thin_issue(const GemmLane<NT>& L, uint8_t* stage, uint32_t c) {
+    using T = ThinLds<SYM, NT>;
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+        lds_buf16(L.abuf, L.a_off[i], c * (kGemmKC * 2u), stage + L.wave * 1024u + (uint32_t)i * 4096u);
+    uint8_t* b = stage + T::kB + L.wave * kGemmBWave;
+    lds_buf16(L.wbuf, L.w_off[0], c * (kGemmKC / 2u), b);
+    lds_buf16(L.wbuf, L.w_off[1], c * (kGemmKC / 2u), b + kGemmBTile);
+    // lane l brings the dword with the chunk's group(s) of its row: row l % 32
+    // of tile l / 32
+    const bool t1 = (threadIdx.x & 32u) != 0u;
+    const uint32_t s = t1 ? L.s_own[1] : L.s_own[0], z = t1 ? L.z_own[1] : L.z_own[0];
+    const uint32_t at = c * (G == 32 ? 4u : 2u);
+    lds_buf4(L.sbuf, G == 32 ? s + at : (s + at) & ~3u, 0u, stage + T::kS + L.wave * 256u);
+    if constexpr (!SYM)
+        lds_buf4(L.zbuf, G == 32 ? z + at : (z + at) & ~3u, 0u, stage + T::kZ + L.wave * 256u);
+}
+
+// a_rd, b_rd: the lane's read addresses of step 0's activations (slice 0) and
+// of its weights in stage 0; tile: the weight tile of slot 0 (HALF: 1 on the
+// waves that run the up rows).
+template <int G, bool SYM, int NT, bool HALF>
+__device__ __forceinline__ void thin_kloop(const GemmLane<NT>& L, uint8_t* smem, uint32_t a_rd,
+                                           uint32_t b_rd, uint32_t tile, f16v_t (&acc)[NT][2]) {
+    using T = ThinLds<SYM, NT>;
+    constexpr uint32_t kLoads = (uint32_t)NT + (SYM ? 3u : 4u);
+    const uint32_t last = L.nchunks - 1u;
+    // chunks past the last repeat it: every chunk issues the same loads
+#pragma unroll
+    for (uint32_t q = 0; q < T::kStages - 1u; ++q)
+        thin_issue<G, SYM, NT>(L, smem + q * T::kStage, q < last ? q : last);
+    const uint32_t m = threadIdx.x & 31u, h = (threadIdx.x >> 5) & 1u;
+    const uint32_t s_rd = lds_addr(smem) + T::kS + L.wave * 256u + (32u * tile + m) * 4u;
+    uint32_t read = 0u, write = (T::kStages - 1u) * T::kStage;  // stages of chunk c and the one issued
+#pragma unroll 1
+    for (uint32_t c = 0; c < L.nchunks; ++c) {
+        wait_vmcnt<(T::kStages - 2u) * kLoads>();
+        block_barrier();
+        const uint32_t ahead = c + T::kStages - 1u;
+        thin_issue<G, SYM, NT>(L, smem + write, ahead < last ? ahead : last);
+        u32x4_t af[2][NT], bw0, bw1;
+        const uint32_t a = a_rd + read, b = b_rd + read;
+        lds_read_act<NT, 0u>(af[0], a);
+        bw0 = lds_read16<0>(b);
+        bw1 = HALF ? bw0 : lds_read16<kGemmBTile>(b);
+        // G = 32: half h takes the dword's group 2 c + h; G = 64: the half
+        // that the row's alignment puts the group in
+        const uint32_t sh0 = G == 32 ? 2u * h : (L.s_own[0] + 2u * c) & 2u;
+        const uint32_t sh1 = G == 32 ? 2u * h : (L.s_own[1] + 2u * c) & 2u;
+        uint32_t s0 = lds_read_u16(s_rd + read + sh0);
+        uint32_t s1 = HALF ? s0 : lds_read_u16(s_rd + read + 128u + sh1);
+        uint32_t z0 = 0u, z1 = 0u;
+        if constexpr (!SYM) {
+            const uint32_t zh0 = G == 32 ? 2u * h : (L.z_own[0] + 2u * c) & 2u;
+            const uint32_t zh1 = G == 32 ? 2u * h : (L.z_own[1] + 2u * c) & 2u;
+            z0 = lds_read_u16(s_rd + read + (T::kZ - T::kS) + zh0);
+            z1 = HALF ? z0 : lds_read_u16(s_rd + read + (T::kZ - T::kS) + 128u + zh1);
+        }
+        lds_wait<NT>(af[0], bw0, bw1, s0, s1, z0, z1);
+        const GroupScale g0 = group_scale<SYM>((uint16_t)s0, (uint16_t)z0);
+        const GroupScale g1 = group_scale<SYM>((uint16_t)s1, (uint16_t)z1);
+#pragma unroll
+        for (int st = 0; st < 4; ++st) {
+            if (st < 3) lds_read_act<NT, 0u>(af[(st + 1) & 1], step_addr(a, (uint32_t)(st + 1)));
+            const h8v_t w0 = dequant8<SYM>(bw0[st], g0), w1 = HALF ? w0 : dequant8<SYM>(bw1[st], g1);
+#pragma unroll
+            for (int i = 0; i < NT; ++i) {
+                const h8v_t x = __builtin_bit_cast(h8v_t, af[st & 1][i]);
+                acc[i][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x, w0, acc[i][0], 0, 0, 0);
+                if constexpr (!HALF)
+                    acc[i][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x, w1, acc[i][1], 0, 0, 0);
+            }
+            if (st < 3) lds_wait<NT>(af[(st + 1) & 1]);
+        }
+        read = read == (T::kStages - 1u) * T::kStage ? 0u : read + T::kStage;
+        write = write == (T::kStages - 1u) * T::kStage ? 0u : write + T::kStage;
+    }
+}
+
 // MODE 0: gate/up + activation; MODE 1: down + scatter; MODE 2: dense
 // projection y[t, n] (the down sub-tensor's geometry, rows taken in order).
 // HALF, dense GEMM: a 128-column tile, wave w the 32 weight rows 32 w .. of
@@ -509,12 +609,12 @@ __host__ __device__ constexpr uint32_t gemm_rows() { return MODE == 2 ? kDenseRo
 template <bool SYM>
 __host__ __device__ constexpr uint32_t next_word() { return GemmLds<kGemmRows>::kWord; }
 
-template <int G, bool SYM, int ACT, int MODE, int NT, bool HALF>
+template <int G, bool SYM, int ACT, int MODE, int NT, bool HALF, bool THIN = false>
 __device__ __forceinline__ void gemm_block(const GemmArgs& args, const tsg_routed_block& blk,
                                            uint32_t rows, uint32_t tile, uint8_t* smem,
                                            bool post, uint32_t next) {
     static_assert(!HALF || MODE != 1, "the down GEMM has no half tiles");
-    constexpr uint32_t R = gemm_rows<MODE>();
+    constexpr uint32_t R = THIN ? kThinRows : gemm_rows<MODE>();
     using Y = GemmLds<R>;
     static_assert(NT >= 1 && (uint32_t)NT <= Y::kSlices, "slices per pass");
     const uint32_t lane = threadIdx.x & 63u, h = lane >> 5, m = lane & 31u;
@@ -624,7 +724,12 @@ __device__ __forceinline__ void gemm_block(const GemmArgs& args, const tsg_route
         const tsg_token_expert_pair pr = args.pairs[blk.pair_start + threadIdx.x];
         row_dst = (pr.token * args.top_k + pr.rank) * args.d;
     }
-    gemm_kloop<R, G, SYM, NT, HALF>(L, smem, acc);
+    if constexpr (THIN) {
+        const uint32_t up = MODE == 0 && HALF && L.wave >= 2u ? 1u : 0u;
+        thin_kloop<G, SYM, NT, HALF>(L, smem, L.a_rd, L.b_rd - Y::kBBase + ThinLds<SYM, NT>::kB, up, acc);
+    } else {
+        gemm_kloop<R, G, SYM, NT, HALF>(L, smem, acc);
+    }
     wait_vmcnt<0>();  // no LDS write may land after this point
 
     // Output: the block's tile goes through LDS (idle now) so
@@ -853,6 +958,47 @@ __device__ __forceinline__ void gemm_item(const GemmArgs& args, const tsg_routed
     }
 }
 
+// The routed GEMMs of a call whose experts have few rows each, in passes of
+// kThinRows rows. Such a call is bound by latency: a weight is dequantised for
+// one or two MFMAs, so a chunk is barrier, LDS reads, dequantisation and MFMAs
+// in turn (0.5 us alone), and two workgroups per CU, which is what the wide
+// kernels' accumulators and rings allow, hide little of it. With a third of
+// the LDS and at most 168 registers three fit. Gate/up and down of 67 tokens,
+// 8 of 128 experts, 2816 x 704: 126 us in the fused launch, 99 here (104 with
+// two per CU and deeper rings, 100 with four and shallower ones; 121 with
+// passes of 32 rows); of 32 tokens 102 and 83; of 9 tokens 86 and 51. Grid:
+// x = items as in moe_gemm_kernel, y = the passes side by side.
+template <int G, bool SYM, int ACT, int MODE>
+__global__ __launch_bounds__(kGemmThreads, 3) void moe_gemm_thin_kernel(GemmArgs args) {
+    extern __shared__ __align__(16) uint8_t smem[];  // kThinLds
+    const uint32_t nb = args.n_blocks_device ? min(*args.n_blocks_device, args.n_blocks) : args.n_blocks;
+    if (blockIdx.x >= nb * args.ntiles) return;
+    uint32_t yb, tile;
+    gemm_work_item(args, nb, blockIdx.x, reinterpret_cast<uint32_t*>(smem), true, yb, tile);
+    const tsg_routed_block blk = args.blocks[yb];
+    // a block list written on the device is not checked on the host: an
+    // expert past the layer is skipped (its weights would lie outside it)
+    if (blk.local_slot >= args.num_experts) {
+        if (blk.row_count != 0 && threadIdx.x == 0) atomicOr(args.error, kErrGemmBlock);
+        return;
+    }
+    const bool half = MODE == 0 && args.f - tile * 128u <= 64u;
+    for (uint32_t r0 = blockIdx.y * kThinRows; r0 < blk.row_count; r0 += gridDim.y * kThinRows) {
+        if (r0 != blockIdx.y * kThinRows) lds_barrier();  // every wave is done with the previous pass's LDS
+        tsg_routed_block sub = blk;
+        sub.pair_start += r0;
+        sub.local_row += r0;
+        const uint32_t rows = blk.row_count - r0 < kThinRows ? blk.row_count - r0 : kThinRows;
+        if (rows > 32u) {
+            if (half) gemm_block<G, SYM, ACT, MODE, 2, MODE == 0, true>(args, sub, rows, tile, smem, false, 0u);
+            else gemm_block<G, SYM, ACT, MODE, 2, false, true>(args, sub, rows, tile, smem, false, 0u);
+        } else {
+            if (half) gemm_block<G, SYM, ACT, MODE, 1, MODE == 0, true>(args, sub, rows, tile, smem, false, 0u);
+            else gemm_block<G, SYM, ACT, MODE, 1, false, true>(args, sub, rows, tile, smem, false, 0u);
+        }
+    }
+}
+
 // 1-D grid of ntiles x (routed block capacity) workgroups; those past the
 // live count exit at once. Two workgroups per CU.
 template <int G, bool SYM, int ACT, int MODE>
@@ -980,12 +1126,42 @@ __global__ __launch_bounds__(kGemmThreads, 2) void moe_gemm_fused_kernel(GemmArg
 
 // ------------------------------------------------------------- launchers
 
+// Whether a device-written work list goes to the thin kernels. The host knows
+// of it only its capacity: of tsg_prefill_group_pairs_device's ceil(pairs /
+// 128) + E entries, those past E count the pairs. 16 are 2048 pairs: gate/up
+// and down of 256 tokens, 2816 x 704, 128 experts, are 192 us fused and 182
+// thin, of 400 tokens 197 and 225 (256 experts of 2048 x 512: 141 and 127, 153
+// and 176 at 509; 32 experts: 115 and 97 at 300). The affine kernels read the
+// zero points too and hold 150 registers: 67 tokens are 135 and 109, 128
+// tokens 162 and 171, so their line is 6, 768 pairs. With three workgroups per
+// CU, each on part of 256 weight rows' lines, wider experts outgrow the L2:
+// 40 tokens of 2048 x 1024 are 124 and 98, of 4096 x 1536 237 and 253 (affine
+// 271 and 361), so d * f stays at 2^21 (2816 x 704 is 1.98 M). A list with
+// spare capacity goes to the wide kernels, with the same results.
+template <bool SYM>
+inline bool few_rows(const GemmArgs& a, uint32_t max_blocks) {
+    return a.n_blocks_device && max_blocks <= (uint64_t)a.num_experts + (SYM ? 16u : 6u) &&
+           (uint64_t)a.d * a.f <= 1u << 21;
+}
+
+template <int G, bool SYM, int MODE>
+tsg_status launch_thin(const tsg_moe* moe, hipStream_t s, const GemmArgs& args, uint32_t max_blocks) {
+    auto kern = moe->activation == TSG_ACT_SILU ? moe_gemm_thin_kernel<G, SYM, TSG_ACT_SILU, MODE>
+                                                : moe_gemm_thin_kernel<G, SYM, TSG_ACT_GELU_TANH, MODE>;
+    // blocks of up to two passes (what the device grouping writes at most)
+    // run them side by side
+    const dim3 grid(args.ntiles * max_blocks, 2u);
+    hipLaunchKernelGGL(kern, grid, dim3(kGemmThreads), kThinLds, s, args);
+    return check_launch(MODE == 0 ? "moe_gemm thin gate/up" : "moe_gemm thin down");
+}
+
 template <int G, bool SYM, int MODE>
 tsg_status launch_gemm(const tsg_moe* moe, hipStream_t s, const GemmArgs& a, uint32_t max_blocks) {
     GemmArgs args = a;
     args.ntiles = MODE == 0 ? (a.f + 127u) / 128u : (a.d + 255u) / 256u;  // 4 waves x 32 / 64 rows
     TSG_REQUIRE((uint64_t)args.ntiles * max_blocks <= 0x7FFFFFFFu, TSG_ERR_INVALID_ARGUMENT,
                 "moe_gemm: %u routed blocks x %u tiles exceed the grid", max_blocks, args.ntiles);
+    if (MODE != 2 && few_rows<SYM>(args, max_blocks)) return launch_thin<G, SYM, MODE>(moe, s, args, max_blocks);
     const dim3 grid(args.ntiles * max_blocks);
     auto kern = moe->activation == TSG_ACT_SILU ? moe_gemm_kernel<G, SYM, TSG_ACT_SILU, MODE>
                                                 : moe_gemm_kernel<G, SYM, TSG_ACT_GELU_TANH, MODE>;
@@ -1000,6 +1176,10 @@ tsg_status launch_gemm(const tsg_moe* moe, hipStream_t s, const GemmArgs& a, uin
 template <int G, bool SYM>
 tsg_status launch_fused(const tsg_moe* moe, hipStream_t s, GemmArgs gu, GemmArgs dn,
                         uint32_t max_blocks) {
+    if (few_rows<SYM>(gu, max_blocks)) {
+        const tsg_status st = launch_gemm<G, SYM, 0>(moe, s, gu, max_blocks);
+        return st ? st : launch_gemm<G, SYM, 1>(moe, s, dn, max_blocks);
+    }
     gu.ntiles = (gu.f + 127u) / 128u;
     dn.ntiles = (dn.d + 255u) / 256u;
     const tsg_ctx* ctx = moe->ctx;
