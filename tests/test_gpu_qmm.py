@@ -98,3 +98,33 @@ def test_qmm_errors(tsg):
         q.encode(w, s, s, x, y, 0, 64, 256)
     assert e.value.status == 1
     ctx.close()
+
+
+@pytest.mark.parametrize("g,scheme", [(32, "sym"), (64, "affine")])
+@pytest.mark.parametrize("t,n,k", [(300, 8192, 2048), (300, 8192, 704)])
+def test_qmm_tables_at_the_end_of_an_allocation(tsg, t, n, k, g, scheme):
+    """The scale and bias tables end where their allocations end (whole 2 MiB
+    pages of their own): the last weight row's windows, which reach past its
+    groups, read nothing behind the table."""
+    import torch
+    print(f"qmm tables at the end t={t} n={n} k={k} g{g} {scheme}", flush=True)
+    sym = scheme == "sym"
+    ctx = tsg.Context(0, group_size=g)
+    ctx.set_affine_scheme(scheme)
+    rng = np.random.default_rng(k + g)
+    packed, scales, biases = operands(rng, n, k, g)
+    xb = oracle.f16_bits(rng.normal(0, 1, t * k).astype(np.float32))
+
+    def at_end(bits):
+        page = torch.zeros(12 << 20, dtype=torch.uint8, device="cuda")
+        tail = page[page.numel() - bits.nbytes:]
+        tail.copy_(torch.from_numpy(np.ascontiguousarray(bits).view(np.uint8).copy()))
+        return tail
+
+    y = empty(t * n)
+    tsg.PrefillInt4QMM(ctx).encode(dev(packed), at_end(scales), None if sym else at_end(biases),
+                                   dev(xb), y, t, n, k)
+    ref = oracle.int4_qmm(packed, scales, None if sym else biases, xb, t, n, k, g, sym)
+    assert oracle.relative_error(oracle.f16_to_float(host(y, np.uint16)),
+                                 oracle.f16_to_float(ref.ravel())) <= kc.NORTH_STAR
+    ctx.close()

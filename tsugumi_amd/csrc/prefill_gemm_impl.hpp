@@ -255,9 +255,12 @@ __device__ __forceinline__ void window_piece(const GemmLane<NT>& L, uint8_t* sme
     uint8_t* dst = smem_sbase + (V & 1u) * kGemmSBuf + L.wave * kGemmSWave + q * 256u;
     const uint32_t srow = q >= 2u ? L.s_ld[1] : L.s_ld[0];
     const uint32_t zrow = q >= 2u ? L.z_ld[1] : L.z_ld[0];
+    // the whole offset in the VGPR: the buffer's range check need not see a
+    // uniform one
     if constexpr (G == 32) {
-        lds_buf4(L.sbuf, srow, (q & 1u) * L.s_q1 + 16u * V, dst);
-        if constexpr (!SYM) lds_buf4(L.zbuf, zrow, (q & 1u) * L.s_q1 + 16u * V, dst + 2u * kGemmSBuf);
+        const uint32_t at = (q & 1u) * L.s_q1 + 16u * V;
+        lds_buf4(L.sbuf, srow + at, 0u, dst);
+        if constexpr (!SYM) lds_buf4(L.zbuf, zrow + at, 0u, dst + 2u * kGemmSBuf);
     } else {
         const uint32_t d4 = 4u * (lane & 3u);
         lds_buf4(L.sbuf, ((srow + (q & 1u) * L.s_q1 + 8u * V) & ~3u) + d4, 0u, dst);
@@ -623,14 +626,16 @@ __device__ __forceinline__ void gemm_block(const GemmArgs& args, const tsg_route
     const uint32_t K = MODE == 0 ? args.d : args.f;
     L.nchunks = K / kGemmKC;
     const uint8_t* blob = args.layer_base + (uint64_t)blk.local_slot * args.expert_stride;
-    // routed GEMMs: loads past the expert's stride read zero (a window past
-    // the last row of the last expert), never another allocation
+    // loads past the expert's stride, or past the dense scale and bias tables
+    // (d x K / G, the launch checks that n * k / 2 fits 32 bits), read zero (a
+    // window past the last row), never another allocation
     const uint32_t wlim = MODE == 2 ? 0xFFFFFFFFu
                                     : (uint32_t)(args.expert_stride < 0xFFFFFFFFull ? args.expert_stride
                                                                                     : 0xFFFFFFFFull);
+    const uint32_t slim = MODE == 2 ? args.d * (K / G) * 2u : wlim;
     L.wbuf = raw_rsrc(blob, wlim);
-    L.sbuf = raw_rsrc(MODE == 2 ? args.dense_s : blob, wlim);
-    L.zbuf = raw_rsrc(MODE == 2 ? args.dense_b : blob, wlim);
+    L.sbuf = raw_rsrc(MODE == 2 ? args.dense_s : blob, slim);
+    L.zbuf = raw_rsrc(MODE == 2 ? args.dense_b : blob, slim);
     L.abuf = raw_rsrc(args.a, 0xFFFFFFFFu);
 
     // the wave's weight rows: tile t row r is row0[t] + r of sub-tensor t
