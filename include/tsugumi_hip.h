@@ -667,7 +667,8 @@ tsg_status tsg_prefill_moe_reduce_token_major(tsg_ctx* ctx, tsg_stream stream,
  * y[t, n] = half(sum_k x[t, k] * half(dequant(W[n, k]))), fp32 accumulation.
  * W is [n, k/2] bytes, scales and biases [n, k/group] bf16 (biases unused
  * under sym). The dequant-to-LDS MFMA GEMM of the routed experts, rows taken
- * in order. Errors: K % group != 0 (the reference's precondition). Declined
+ * in order; few workgroups' worth of rows and columns split K over waves
+ * instead (fp32 partial sums, a fixed order for a given t, n and k). Errors: K % group != 0 (the reference's precondition). Declined
  * with TSG_ERR_UNSUPPORTED: K or N not a multiple of 64, t*n or t*k >= 2^32,
  * or W of 4 GiB or more. */
 tsg_status tsg_prefill_int4_qmm(tsg_ctx* ctx, tsg_stream stream, const uint8_t* weights,

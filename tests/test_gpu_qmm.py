@@ -128,3 +128,37 @@ def test_qmm_tables_at_the_end_of_an_allocation(tsg, t, n, k, g, scheme):
     assert oracle.relative_error(oracle.f16_to_float(host(y, np.uint16)),
                                  oracle.f16_to_float(ref.ravel())) <= kc.NORTH_STAR
     ctx.close()
+
+
+@pytest.mark.parametrize("g,scheme", [(32, "sym"), (32, "affine"), (64, "sym"), (64, "affine")])
+@pytest.mark.parametrize("t,n,k", [(1, 64, 64), (31, 64, 448), (32, 128, 512), (33, 192, 576),
+                                   (65, 64, 2112), (67, 4096, 2816)])
+def test_qmm_of_few_rows(tsg, t, n, k, g, scheme):
+    """The K-split kernel at the edges of its row blocks (1 to 67 rows) and of
+    its deal of chunks (fewer than the waves, one round, one more, the read-ahead
+    and past it), against fp64 over the kernel's fp16 weights: one fp16 rounding
+    of each result (2^-11 of it) and K fp32 roundings (K 2^-24 of the sum of
+    the magnitudes). The rows past y keep their bytes."""
+    print(f"qmm few rows t={t} n={n} k={k} g{g} {scheme}", flush=True)
+    sym = scheme == "sym"
+    ctx = tsg.Context(0, group_size=g)
+    ctx.set_affine_scheme(scheme)
+    rng = np.random.default_rng(t + n + k)
+    packed, scales, biases = operands(rng, n, k, g)
+    xb = oracle.f16_bits(rng.normal(0, 1, t * k).astype(np.float32))
+    y = empty(t * n + 64, fill=0x1234)
+    tsg.PrefillInt4QMM(ctx).encode(dev(packed), dev(scales), None if sym else dev(biases),
+                                   dev(xb), y, t, n, k)
+    got = host(y, np.uint16)
+    assert np.all(got[t * n:] == 0x1234)
+    s = np.repeat(oracle.bf16_to_float(scales).reshape(n, k // g).astype(np.float32), g, axis=1)
+    b = (np.float32(-8) * s if sym else
+         np.repeat(oracle.bf16_to_float(biases).reshape(n, k // g).astype(np.float32), g, axis=1))
+    q = np.stack([packed & 15, packed >> 4], axis=-1).reshape(n, k)
+    # q s is exact in fp64, q s + b rounds there before fp32: twice, at most 1 ulp
+    w = (q.astype(np.float64) * s + b).astype(np.float32).astype(np.float16).astype(np.float64)
+    x = oracle.f16_to_float(xb).reshape(t, k).astype(np.float64)
+    ref, mag = x @ w.T, np.abs(x) @ np.abs(w).T
+    err = np.abs(oracle.f16_to_float(got[:t * n]).reshape(t, n) - ref)
+    assert np.all(err <= np.abs(ref) * 2.0 ** -11 + mag * k * 2.0 ** -24 + 2.0 ** -25)
+    ctx.close()

@@ -1207,9 +1207,104 @@ tsg_status launch_fused(const tsg_moe* moe, hipStream_t s, GemmArgs gu, GemmArgs
 
 // Dense projection: blocks of kDenseRows (128) rows of x in order, 256
 // output columns per workgroup (the down GEMM's tiling).
+// The dense projection of few rows: 32 rows x 32 weight rows a workgroup, the
+// chunks of K dealt to its kSplitWaves waves, whose fp32 accumulators are
+// added in wave order through LDS. With 128 columns a workgroup, 67 rows x 4096
+// columns are 32 workgroups on 256 CUs, each a chain of K / 64 chunks of
+// 0.5 us; here they are 384 with an eighth of the chain and no barrier in it,
+// the operands in registers three chunks ahead. Bound by the L1: a lane reads
+// its own row, so a load touches 32 lines. K = 2816: 67 x 4096 24.9 -> 17.2 us,
+// 9 rows 20.5 -> 7.9, 704 columns of 256 rows 29.5 -> 11.8.
+constexpr uint32_t kSplitWaves = 8;
+
+// One lane's operands of a chunk: K 64 c + 32 h .. + 32 of its activation row
+// and of its weight row, and their group's parameters.
+struct SplitFrag {
+    u32x4_t w, a[4];
+    uint16_t s, z;
+};
+
+template <int G, bool SYM>
+__global__ __launch_bounds__(64u * kSplitWaves, 4) void qmm_split_kernel(GemmArgs args) {
+    __shared__ float part[kSplitWaves][16][64];
+    const uint32_t lane = threadIdx.x & 63u, h = lane >> 5, m = lane & 31u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t K = args.f, n = K / kGemmKC;
+    const uint32_t col = 32u * blockIdx.x + m, row0 = 32u * blockIdx.y;
+    const uint32_t rows = args.dense_rows - row0 < 32u ? args.dense_rows - row0 : 32u;
+    const uint8_t* wp = args.layer_base + (uint64_t)col * (K / 2u) + 16u * h;
+    const uint16_t* ap = args.a + (uint64_t)(row0 + (m < rows ? m : 0u)) * K + 32u * h;
+    const uint16_t* sp = reinterpret_cast<const uint16_t*>(args.dense_s) + (uint64_t)col * (K / G);
+    const uint16_t* zp = reinterpret_cast<const uint16_t*>(args.dense_b) + (uint64_t)col * (K / G);
+    auto load = [&](uint32_t c) {
+        c = c < n ? c : n - 1u;
+        SplitFrag f;
+        f.w = *reinterpret_cast<const u32x4_t*>(wp + c * (kGemmKC / 2u));
+#pragma unroll
+        for (int st = 0; st < 4; ++st)
+            f.a[st] = *reinterpret_cast<const u32x4_t*>(ap + c * kGemmKC + 8u * st);
+        const uint32_t g = G == 32 ? 2u * c + h : c;
+        f.s = sp[g];
+        f.z = SYM ? (uint16_t)0 : zp[g];
+        return f;
+    };
+    constexpr uint32_t kAhead = 3u;
+    SplitFrag q[kAhead];
+#pragma unroll
+    for (uint32_t j = 0; j < kAhead; ++j) q[j] = load(wave + j * kSplitWaves);
+    f16v_t acc = f16v_t{};
+#pragma unroll 1
+    for (uint32_t c = wave; c < n; c += kAhead * kSplitWaves) {
+#pragma unroll
+        for (uint32_t j = 0; j < kAhead; ++j) {
+            if (c + j * kSplitWaves < n) {
+                const GroupScale g = group_scale<SYM>(q[j].s, q[j].z);
+#pragma unroll
+                for (int st = 0; st < 4; ++st)
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8v_t, q[j].a[st]),
+                                                                 dequant8<SYM>(q[j].w[st], g), acc, 0, 0, 0);
+            }
+            q[j] = load(c + (kAhead + j) * kSplitWaves);
+        }
+    }
+#pragma unroll
+    for (int v = 0; v < 16; ++v) part[wave][v][lane] = acc[v];
+    __syncthreads();
+    // acc[v] of lane (h, m): row 8 (v / 4) + 4 h + v % 4, column m
+    const uint32_t r = threadIdx.x >> 4, c2 = 2u * (threadIdx.x & 15u);
+    if (r >= rows) return;
+    const uint32_t v = ((r >> 3) << 2) | (r & 3u), l = 32u * ((r >> 2) & 1u) + c2;
+    float y0 = 0.0f, y1 = 0.0f;
+#pragma unroll
+    for (uint32_t w = 0; w < kSplitWaves; ++w) {
+        y0 += part[w][v][l];
+        y1 += part[w][v][l + 1u];
+    }
+    *reinterpret_cast<uint32_t*>(args.out + (uint64_t)(row0 + r) * args.d + 32u * blockIdx.x + c2) =
+        (uint32_t)f32_to_f16(y0) | (uint32_t)f32_to_f16(y1) << 16;
+}
+static_assert(64u * kSplitWaves == 32u * 16u, "one thread per pair of outputs");
+
 template <int G, bool SYM>
 tsg_status launch_dense_qmm(hipStream_t s, const GemmArgs& a, uint32_t num_cus) {
     GemmArgs args = a;
+    // Few workgroups: the K split. Its time goes in steps of a workgroup per CU
+    // (11.5 us at K = 2816, 12.4 at 2048, 6.8 at 704), the GEMM's hardly grows
+    // until its own grid fills the device. One step is always the faster (2048 x
+    // 2048, 128 rows: 22.8 and 12.7; 1024 x 704, 256 rows: 10.8 and 7.1); two are
+    // where K is long (4096 x 2816, 128 rows: 29.8 and 21.6; 2816 x 4096: 41.0
+    // and 30.7; but 2048 x 2048, 256 rows: 23.0 and 23.3, affine 27.0; 1024 x
+    // 704, 320 rows: 10.8 and 11.9), three nowhere (4096 x 2816, 160 rows: 29.9
+    // and 30.8). A y that overlaps x keeps the GEMM's order of reads and writes.
+    const uint64_t split = (uint64_t)(a.d / 32u) * ((a.dense_rows + 31u) / 32u);
+    const uintptr_t x0 = reinterpret_cast<uintptr_t>(a.a), y0 = reinterpret_cast<uintptr_t>(a.out);
+    const bool apart = x0 + (uint64_t)a.dense_rows * a.f * 2u <= y0 ||
+                       y0 + (uint64_t)a.dense_rows * a.d * 2u <= x0;
+    if (split <= (a.f > 2048u ? 2u : 1u) * num_cus && apart) {
+        hipLaunchKernelGGL((qmm_split_kernel<G, SYM>), dim3(a.d / 32u, (a.dense_rows + 31u) / 32u),
+                           dim3(64u * kSplitWaves), 0, s, args);
+        return check_launch("qmm split");
+    }
     args.n_blocks = (a.dense_rows + kDenseRows - 1u) / kDenseRows;
     // 256-column tiles while they cover the device's CUs; below that, 128-column
     // tiles (one 32-row weight tile per wave, the same MFMA sequence per
