@@ -603,7 +603,9 @@ tsg_status tsg_prefill_moe_down(tsg_moe* moe, tsg_stream stream, const tsg_layer
  * the two encodes the reference issues back to back) in one persistent
  * launch: exactly tsg_prefill_moe_gate_up followed by tsg_prefill_moe_down on
  * the same arguments (bit-identical act and route_partials), with the down
- * tiles of a block starting as soon as that block's gate/up tiles are done.
+ * tiles of a block starting as soon as that block's gate/up tiles are done;
+ * a device-counted list whose capacity n_blocks is at most the experts and a
+ * few (few rows an expert) runs as two launches instead, with the same bits.
  * The reference has no single call for the pair; a caller that issues the two
  * encodes back to back replaces them with this one. act must be 128-byte
  * aligned (TSG_ERR_ALIGNMENT); at most 65536 blocks. The schedule words live

@@ -727,8 +727,8 @@ class PrefillGroupedRoutedMoE:
     def encode_gate_up_down(self, layer, hidden, hidden_stride, sorted_pairs, blocks, n_blocks,
                             act, route_partials, top_k, d, f, n_blocks_device=None,
                             stream=None):
-        """encode_gate_up then encode_down in one persistent launch (same
-        results; act 128-byte aligned)."""
+        """encode_gate_up then encode_down in one call (same results; act
+        128-byte aligned): one persistent launch, two for few rows an expert."""
         check(self.lib.tsg_prefill_moe_gate_up_down(
             self.moe.handle, _stream(stream), layer.handle, _ptr(hidden), hidden_stride,
             _ptr(sorted_pairs), _ptr(blocks), n_blocks, _ptr(n_blocks_device), _ptr(act),
