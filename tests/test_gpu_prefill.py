@@ -196,6 +196,41 @@ def test_device_grouping_matches_host_sort(tsg, ctx, t, ne, k, s, tile):
     assert np.all(covered == 1)
 
 
+@pytest.mark.parametrize("t,ne,k,tile", [(1, 1, 1, 32), (1, 128, 8, 128), (8, 255, 8, 64),
+                                         (13, 9, 5, 32), (128, 256, 8, 128), (1025, 1, 1, 32),
+                                         (67, 128, 8, 256), (682, 8, 3, 64), (256, 256, 8, 256),
+                                         (2048, 2, 1, 32), (2049, 2, 1, 32)])
+def test_small_device_grouping_matches_host_sort(tsg, ctx, t, ne, k, tile):
+    """One workgroup up to 2048 pairs: a lane, a wave and a step more or less,
+    one expert and 256, lists of full blocks and of remainders; largest first."""
+    test_device_grouping_matches_host_sort(tsg, ctx, t, ne, k, 1.0, tile)
+    rng = np.random.default_rng(t + ne)
+    idx = _zipf_routing(rng, t, ne, k, 1.0)[0].reshape(-1)
+    idx[rng.random(t * k) < 0.1] = ne  # left out, and reported
+    w = np.arange(t * k, dtype=np.uint16)
+    max_blocks = t * k // tile + ne + 1
+    sp, off, cnt = empty(t * k * 4, np.uint32), empty(ne, np.uint32), empty(ne, np.uint32)
+    blocks, nb = empty(max_blocks * 4, np.uint32), empty(1, np.uint32)
+    g = tsg.PrefillGroupedRoutedMoE(tsg.MoE(ctx))
+    g.group_pairs_device(dev(idx), dev(w), t, k, ne, sp, off, cnt, blocks, max_blocks, nb,
+                         empty(g.scratch_bytes(t, k, ne) // 4 + 1, np.uint32), tile_rows=tile)
+    if (idx == ne).any():
+        with pytest.raises(tsg.TsgError):
+            ctx.synchronize()
+    order = np.argsort(idx, kind="stable")[:int((idx < ne).sum())]
+    got = host(sp, np.uint32).view(oracle.PAIR_DTYPE)[:len(order)]
+    assert np.array_equal(got["token"] * k + got["rank"], order)
+    assert np.array_equal(got["expert"], idx[order])
+    assert np.array_equal(got["weight_bits"], w[order])
+    counts = np.bincount(idx[order], minlength=ne)
+    assert np.array_equal(host(cnt, np.uint32), counts)
+    bl = host(blocks, np.uint32).view(oracle.BLOCK_DTYPE)[:int(host(nb, np.uint32)[0])]
+    rows = [(min(c - r, tile), e, r) for e, c in enumerate(counts) for r in range(0, c, tile)]
+    rows.sort(key=lambda b: (-min(-(-b[0] // 32), 8), b[1], b[2]))
+    first = np.cumsum(counts) - counts
+    assert [tuple(b) for b in bl] == [(e, first[e] + r, n, first[e] + r) for n, e, r in rows]
+
+
 def test_rows_path_matches_decode_bitwise(tsg, ctx):
     """PrefillRoutedMoERowsVsDecodeTests.swift:23-166: one token routed to all
     eight experts; rows-path activations equal decode phase 1's bit for bit,

@@ -178,6 +178,153 @@ __global__ __launch_bounds__(256) void group_scatter_kernel(
     }
 }
 
+// The whole grouping of a call of few pairs in one workgroup, nothing through
+// memory. Bound by latency: the two launches above are a launch, a read of the
+// ids, a scan, and all of that again. Each wave owns `per` consecutive pairs
+// (64 a step): a lane's rank among the step's equal ids comes from ballots of
+// the id's bits, the earlier steps' count from the wave's histogram row, the
+// earlier waves' from the scan over the rows, so the order is (token, rank)
+// as above. The list's eight size buckets are 16-bit fields of two words and
+// take one scan instead of eight. Back to back in a HIP graph, us, two launches
+// and here: 9 tokens of top-8 over 128 experts 8.2 and 4.1, 128 tokens 8.5 and
+// 4.3, 256 8.4 and 5.2. One CU's stores of the pairs grow with their number
+// (400 tokens 8.3 and 7.0, 512 8.3 and 7.4), so the line is at 2048 pairs,
+// below which a whole prompt layer gains what the grouping does (9 tokens 79.6
+// -> 75.2, 128 tokens 167.4 -> 163.1) and above which it did so within noise.
+constexpr uint32_t kSmallPairs = 2048u;
+constexpr uint32_t kSmallThreads = 1024u, kSmallWaves = kSmallThreads / 64u;
+constexpr uint32_t kSmallSteps = kSmallPairs / kSmallThreads;
+static_assert(kSmallPairs / 32u + kMaxExperts < 65536u, "the bucket counts fit 16 bits");
+
+__device__ __forceinline__ uint64_t wave_inclusive_scan64(uint64_t x, uint32_t lane) {
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint64_t o = __shfl_up((unsigned long long)x, off, 64);
+        if ((int)lane >= off) x += o;
+    }
+    return x;
+}
+
+__global__ __launch_bounds__(kSmallThreads) void group_small_kernel(
+    const uint32_t* __restrict__ idx, const uint16_t* __restrict__ w, uint32_t n, uint32_t k,
+    uint32_t ne, tsg_token_expert_pair* __restrict__ sorted, uint32_t* __restrict__ offsets,
+    uint32_t* __restrict__ counts, tsg_routed_block* __restrict__ blocks, uint32_t max_blocks,
+    uint32_t* __restrict__ n_blocks, uint32_t tile_rows, uint32_t* __restrict__ error_word) {
+    static_assert(kMaxExperts <= 256, "eight id bits, one expert per thread of four waves");
+    __shared__ uint32_t hist[kSmallWaves][256];
+    __shared__ uint32_t off_s[256];
+    __shared__ uint64_t tot[4][3];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t per = 64u * ((n + kSmallThreads - 1u) / kSmallThreads);
+    const uint32_t p0 = wave * per + lane, steps = per / 64u;
+    uint32_t ex[kSmallSteps], wt[kSmallSteps], rank[kSmallSteps];
+#pragma unroll
+    for (uint32_t i = 0; i < kSmallSteps; ++i) {
+        const bool in = i < steps && p0 + 64u * i < n;
+        ex[i] = in ? idx[p0 + 64u * i] : 0xFFFFFFFFu;
+        wt[i] = in ? (uint32_t)w[p0 + 64u * i] : 0u;
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < 4u; ++i) hist[wave][64u * i + lane] = 0u;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t i = 0; i < kSmallSteps; ++i) {
+        if (i >= steps) break;
+        const uint32_t id = ex[i];
+        const bool ok = id < ne;
+        uint64_t same = __ballot(ok);
+#pragma unroll
+        for (uint32_t b = 0; b < 8u; ++b) {
+            const bool bit = (id >> b) & 1u;
+            const uint64_t ones = __ballot(bit);
+            same &= bit ? ones : ~ones;
+        }
+        const uint32_t base = ok ? hist[wave][id] : 0u;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        rank[i] = base + (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
+        if (ok && (same >> lane) == 1ull) hist[wave][id] = base + (uint32_t)__popcll(same);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (!ok && p0 + 64u * i < n) atomicOr(error_word, kErrGroupExpertRange);
+    }
+    __syncthreads();
+    // thread e: its expert's count, offset and place in the list
+    const uint32_t e = threadIdx.x;
+    uint32_t c = 0u, full = 0u, rem = 0u, qfull = 0u, qrem = 0u;
+    uint64_t own[3] = {0u, 0u, 0u}, sum[3] = {0u, 0u, 0u};  // buckets 8..5, 4..1, pairs
+    if (e < 256u) {
+#pragma unroll
+        for (uint32_t v = 0; v < kSmallWaves; ++v) {
+            const uint32_t h = hist[v][e];
+            hist[v][e] = c;
+            c += h;
+        }
+        full = c / tile_rows;
+        rem = c - full * tile_rows;
+        qfull = 8u - min(tile_rows / 32u, 8u);
+        qrem = 8u - (rem ? min((rem + 31u) / 32u, 8u) : 8u);
+        const uint64_t vf = (uint64_t)full << (16u * (qfull & 3u));
+        const uint64_t vr = rem ? 1ull << (16u * (qrem & 3u)) : 0ull;
+        own[0] = (qfull < 4u ? vf : 0ull) + (qrem < 4u ? vr : 0ull);
+        own[1] = (qfull < 4u ? 0ull : vf) + (qrem < 4u ? 0ull : vr);
+        own[2] = c;
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            sum[j] = wave_inclusive_scan64(own[j], lane);
+            if (lane == 63u) tot[wave][j] = sum[j];
+        }
+    }
+    __syncthreads();
+    uint32_t off = 0u;
+    uint64_t all[3] = {0u, 0u, 0u};
+    if (e < 256u) {
+#pragma unroll
+        for (uint32_t v = 0; v < 4u; ++v)
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+                const uint64_t x = tot[v][j];
+                sum[j] += v < wave ? x : 0u;
+                all[j] += x;
+            }
+#pragma unroll
+        for (int j = 0; j < 3; ++j) sum[j] -= own[j];
+        off = (uint32_t)sum[2];
+        off_s[e] = off;
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t i = 0; i < kSmallSteps; ++i) {
+        const uint32_t p = p0 + 64u * i;
+        if (i >= steps || ex[i] >= ne) continue;
+        const uint32_t tok = p / k;
+        sorted[off_s[ex[i]] + hist[wave][ex[i]] + rank[i]] =
+            tsg_token_expert_pair{tok, ex[i], p - tok * k, wt[i]};
+    }
+    if (e >= 256u) return;
+    uint32_t first_full = 0u, first_rem = 0u, running = 0u;
+#pragma unroll
+    for (uint32_t q = 0; q < 8u; ++q) {
+        const uint32_t at = running + ((uint32_t)(sum[q >> 2] >> (16u * (q & 3u))) & 0xFFFFu);
+        if (q == qfull) first_full = at;
+        if (q == qrem) first_rem = at + (q == qfull ? full : 0u);
+        running += (uint32_t)(all[q >> 2] >> (16u * (q & 3u))) & 0xFFFFu;
+    }
+    if (e == 0u) {
+        *n_blocks = running < max_blocks ? running : max_blocks;
+        if (running > max_blocks) atomicOr(error_word, kErrGroupBlocks);
+    }
+    if (e >= ne) return;
+    counts[e] = c;
+    offsets[e] = c ? off : 0xFFFFFFFFu;
+    for (uint32_t b = 0; b < full; ++b) {
+        const uint32_t bi = first_full + b, start = off + b * tile_rows;
+        if (bi < max_blocks) blocks[bi] = tsg_routed_block{e, start, tile_rows, start};
+    }
+    if (rem && first_rem < max_blocks) {
+        const uint32_t start = off + full * tile_rows;
+        blocks[first_rem] = tsg_routed_block{e, start, rem, start};
+    }
+}
+
 // ---------------------------------------------------- token-major reduce
 
 __global__ __launch_bounds__(256) void reduce_token_major_kernel(
@@ -508,6 +655,12 @@ tsg_status group_pairs_device(tsg_ctx* ctx, hipStream_t s, const uint32_t* idx,
     TSG_REQUIRE(max_blocks >= need, TSG_ERR_INVALID_ARGUMENT,
                 "max_blocks %u cannot hold the work list: need min(t*k, ceil(t*k/%u) + %u) = %llu",
                 max_blocks, tile_rows, ne, (unsigned long long)need);
+    if (pairs_total <= kSmallPairs) {
+        hipLaunchKernelGGL(group_small_kernel, dim3(1), dim3(kSmallThreads), 0, s, idx, w, t * k, k, ne,
+                           sorted, offsets, counts, blocks, max_blocks, n_blocks, tile_rows,
+                           ctx->counters + kSyncErrorWord);
+        return check_launch("group_small");
+    }
     hipLaunchKernelGGL(group_rank_kernel, dim3(ne), dim3(1024), 0, s, idx, t, k, rank_of, counts);
     tsg_status st = check_launch("group_rank");
     if (st) return st;
