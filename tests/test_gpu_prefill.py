@@ -484,14 +484,14 @@ def test_gate_up_half_tile_equals_full_tile(tsg, ctx, group, scheme):
 
 @pytest.mark.parametrize("group,scheme,act", [(32, "sym", "silu"), (32, "affine", "gelu"),
                                               (64, "sym", "gelu"), (64, "affine", "silu")])
-@pytest.mark.parametrize("d,f", [(512, 704), (320, 64), (64, 192), (832, 128)])
+@pytest.mark.parametrize("d,f", [(512, 704), (320, 64), (64, 192), (832, 128), (1856, 64)])
 def test_few_rows_gemms_equal_the_wide_ones(tsg, ctx, group, scheme, act, d, f):
     """A device work list whose capacity is at most the experts + 6 runs the
     three-per-CU kernels, one with spare capacity the wide ones: the same
     activations and partials, bit for bit, from the one-launch entry and from
     the two separate ones. Blocks of 1 to 200 rows: both slice counts, one to
-    four passes; K of 1 to 13 chunks (shorter than the ring, odd, ragged G = 64
-    windows); half and partial column tiles."""
+    four passes; K of 1 to 29 chunks (shorter than the ring, odd, ragged G = 64
+    windows, every window buffer taken again); half and partial column tiles."""
     sym = scheme == "sym"
     configure(ctx, group, scheme)
     rows = [1, 0, 31, 32, 33, 64, 65, 128, 129, 200]
@@ -525,3 +525,51 @@ def test_few_rows_gemms_equal_the_wide_ones(tsg, ctx, group, scheme, act, d, f):
     assert not np.isnan(out[0][1].view(np.float16)).any()
     for a, p in out[1:]:
         assert np.array_equal(a, out[0][0]) and np.array_equal(p, out[0][1])
+
+
+@pytest.mark.parametrize("ne,d,f,pairs,group,scheme", [(128, 2816, 704, 768, 32, "affine"),
+                                                       (256, 2048, 512, 536, 32, "affine"),
+                                                       (256, 2048, 512, 1024, 32, "sym")])
+def test_few_rows_gemms_keep_up_on_even_routing(tsg, ctx, ne, d, f, pairs, group, scheme):
+    """Routing that reads nearly every expert is where the few-rows kernels
+    once lost to the wide ones they replace: 1.58, 1.55 and 1.25 of their time
+    at these sizes, with a dword of group parameters a weight row and chunk.
+    The windows brought that to 0.95-1.02; 1.15 leaves room for a noisy run.
+    The experts (0.4-0.5 GB) are in no cache."""
+    import torch
+    configure(ctx, group, scheme)
+    sym, k = scheme == "sym", 8
+    t = pairs // k
+    offs, at = [], 0
+    for r, c in ((f, d), (f, d), (d, f)):
+        w_bytes, s_bytes = r * c // 2, r * (c // group) * 2
+        offs += [at, at + w_bytes, at + w_bytes + (0 if sym else s_bytes)]
+        at += w_bytes + s_bytes * (1 if sym else 2)
+    stride = -(-at // 16384) * 16384
+    image = torch.randint(-2**63, 2**63 - 1, (ne * stride // 8,), dtype=torch.int64, device="cuda")
+    layer = tsg.ResidentLayer(ctx, ne, stride, offs, device_tensor=image.view(torch.uint8))
+    rng = np.random.default_rng(pairs)
+    idx = np.argsort(rng.random((t, ne)), axis=1)[:, :k].astype(np.uint32)
+    g = tsg.PrefillGroupedRoutedMoE(tsg.MoE(ctx))
+    tight, spare = -(-pairs // 128) + ne, -(-pairs // 128) + ne + 40
+    sp, nb, blocks = empty(pairs * 4, np.uint32), empty(1, np.uint32), empty(spare * 4, np.uint32)
+    g.group_pairs_device(dev(idx), dev(np.zeros((t, k), np.uint16)), t, k, ne, sp,
+                         empty(ne, np.uint32), empty(ne, np.uint32), blocks, spare, nb,
+                         empty(pairs + 1, np.uint32), tile_rows=128)
+    hidden = dev(wl.f16_normal(rng, t * d))
+    act, part = empty(pairs * f), empty(pairs * d)
+
+    def us(cap):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(10):
+            g.encode_gate_up_down(layer, hidden, d, sp, blocks, cap, act, part, k, d, f,
+                                  n_blocks_device=nb)
+        b.record()
+        b.synchronize()
+        return a.elapsed_time(b) * 100.0
+
+    us(tight), us(spare)
+    few, wide = (min(v) for v in zip(*((us(tight), us(spare)) for _ in range(7))))
+    print(f"E={ne} {d}x{f} g{group} {scheme} {pairs} pairs: few-rows {few:.1f} us, wide {wide:.1f}")
+    assert few <= 1.15 * wide

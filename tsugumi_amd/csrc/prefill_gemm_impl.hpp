@@ -494,82 +494,142 @@ __device__ __forceinline__ void gemm_kloop(const GemmLane<NT>& L, uint8_t* smem,
 
 // ---- the K loop of the thin kernels (passes of at most kThinRows rows)
 //
-// A chunk's activations (NT slices), weights and one dword of group parameters
-// a row share an LDS stage; the loop over chunks is rolled, with the stage as
-// a run-time offset, kStages - 1 chunks ahead (3 of one slice, 2 of two). One
-// barrier a chunk: it publishes chunk c and frees chunk c - 1's stage. Every
-// accumulator sees gemm_kloop's MFMA sequence, so the results are the same.
+// A chunk's activations (NT slices) and weights share an LDS stage; the loop
+// over chunks is rolled, with the stage as a run-time offset, kStages - 1
+// chunks ahead (gate/up: sym 4 of one slice and 3 of two, affine 3 and 2; down:
+// sym 3 and 2, affine 2 and 1). One barrier a chunk: it publishes chunk c and
+// frees chunk c - 1's stage. Every accumulator sees gemm_kloop's MFMA sequence,
+// so the results are the same.
+// Group parameters: a dword a row and chunk is a load of 64 lines for 4 bytes
+// of each, and where K is long those lines and the weights' outgrow the L2
+// before their next dword is read. Gate/up (K = d) therefore takes the wide
+// kernels' 16-byte windows of four chunks, in three buffers past the stages,
+// with two workgroups per CU; down (K = f, whose parameter rows lie a few to a
+// line) the chunk's dword in its stage, with three.
 constexpr uint32_t kThinRows = 64u;
-constexpr uint32_t kThinLds = 53248u;  // three workgroups per CU
-template <bool SYM, int NT>
+__host__ __device__ constexpr uint32_t thin_per_cu(int mode) { return mode == 0 ? 2u : 3u; }
+template <bool SYM, int NT, int MODE>
 struct ThinLds {
+    static constexpr bool kWindows = MODE == 0;
+    static constexpr uint32_t kBytes = MODE == 0 ? 81920u : 53248u;
     static constexpr uint32_t kB = NT * 4096u;                  // after the activations
-    static constexpr uint32_t kS = kB + kGemmBStage;            // 64 rows x 4 bytes a wave
+    static constexpr uint32_t kS = kB + kGemmBStage;            // no windows: 64 rows x 4 bytes a wave
     static constexpr uint32_t kZ = kS + kGemmWaves * 256u;
-    static constexpr uint32_t kStage = kZ + (SYM ? 0u : kGemmWaves * 256u);
-    static constexpr uint32_t kStages = kThinLds / kStage;
+    static constexpr uint32_t kStage = kWindows ? kS : kZ + (SYM ? 0u : kGemmWaves * 256u);
+    static constexpr uint32_t kBufs = 3u;                       // scale windows, then bias windows
+    static constexpr uint32_t kWin = kWindows ? kBufs * kGemmSBuf * (SYM ? 1u : 2u) : 0u;
+    static constexpr uint32_t kStages = (kBytes - kWin) / kStage;
+    static constexpr uint32_t kW = kStages * kStage;            // where the windows start
     static_assert(kStage % 128u == 0 && kStages >= 2u, "ring");
+    static_assert(kBytes * thin_per_cu(MODE) <= 160u * 1024u, "workgroups per CU");
+    static_assert(GemmLds<kThinRows>::kEpi <= kBytes, "epilogue");
+    // chunk c reads its window after its loads are issued: window V last in
+    // chunk 4 V + 3, and the first piece of window V + kBufs goes out in chunk
+    // 4 (V + kBufs) - 3 - (kStages - 1)
+    static_assert(!kWindows || 4u * kBufs > kStages + 5u, "a window is read before it is overwritten");
 };
-static_assert(GemmLds<kThinRows>::kEpi <= kThinLds && 3u * kThinLds <= 160u * 1024u, "three per CU");
 
-template <int G, bool SYM, int NT>
-__device__ __forceinline__ void thin_issue(const GemmLane<NT>& L, uint8_t* stage, uint32_t c) {
-    using T = ThinLds<SYM, NT>;
+// Piece q of window V (window_piece's load) into the buffer at `dst`.
+template <int G, bool SYM, int NT, int MODE>
+__device__ __forceinline__ void thin_window(const GemmLane<NT>& L, uint8_t* dst, uint32_t q, uint32_t V) {
+    using T = ThinLds<SYM, NT, MODE>;
+    const uint32_t row = (q & 1u) * L.s_q1, d4 = 4u * (threadIdx.x & 3u);
+    const uint32_t s = (q >= 2u ? L.s_ld[1] : L.s_ld[0]) + row, z = (q >= 2u ? L.z_ld[1] : L.z_ld[0]) + row;
+    uint8_t* to = dst + L.wave * kGemmSWave + q * 256u;
+    lds_buf4(L.sbuf, G == 32 ? s + 16u * V : ((s + 8u * V) & ~3u) + d4, 0u, to);
+    if constexpr (!SYM)
+        lds_buf4(L.zbuf, G == 32 ? z + 16u * V : ((z + 8u * V) & ~3u) + d4, 0u, to + T::kBufs * kGemmSBuf);
+}
+
+template <int G, bool SYM, int NT, int MODE>
+__device__ __forceinline__ void thin_issue(const GemmLane<NT>& L, uint8_t* smem, uint8_t* stage, uint32_t c) {
+    using T = ThinLds<SYM, NT, MODE>;
 #pragma unroll
     for (int i = 0; i < NT; ++i)
         lds_buf16(L.abuf, L.a_off[i], c * (kGemmKC * 2u), stage + L.wave * 1024u + (uint32_t)i * 4096u);
     uint8_t* b = stage + T::kB + L.wave * kGemmBWave;
     lds_buf16(L.wbuf, L.w_off[0], c * (kGemmKC / 2u), b);
     lds_buf16(L.wbuf, L.w_off[1], c * (kGemmKC / 2u), b + kGemmBTile);
-    // lane l brings the dword with the chunk's group(s) of its row: row l % 32
-    // of tile l / 32
-    const bool t1 = (threadIdx.x & 32u) != 0u;
-    const uint32_t s = t1 ? L.s_own[1] : L.s_own[0], z = t1 ? L.z_own[1] : L.z_own[0];
-    const uint32_t at = c * (G == 32 ? 4u : 2u);
-    lds_buf4(L.sbuf, G == 32 ? s + at : (s + at) & ~3u, 0u, stage + T::kS + L.wave * 256u);
-    if constexpr (!SYM)
-        lds_buf4(L.zbuf, G == 32 ? z + at : (z + at) & ~3u, 0u, stage + T::kZ + L.wave * 256u);
+    if constexpr (T::kWindows) {
+        const uint32_t V = (c + 3u) >> 2;
+        thin_window<G, SYM, NT, MODE>(L, smem + T::kW + V % T::kBufs * kGemmSBuf, (c + 3u) & 3u, V);
+    } else {
+        // lane l brings the dword with the chunk's group(s) of its row: row
+        // l % 32 of tile l / 32
+        const bool t1 = (threadIdx.x & 32u) != 0u;
+        const uint32_t s = t1 ? L.s_own[1] : L.s_own[0], z = t1 ? L.z_own[1] : L.z_own[0];
+        const uint32_t at = c * (G == 32 ? 4u : 2u);
+        lds_buf4(L.sbuf, G == 32 ? s + at : (s + at) & ~3u, 0u, stage + T::kS + L.wave * 256u);
+        if constexpr (!SYM)
+            lds_buf4(L.zbuf, G == 32 ? z + at : (z + at) & ~3u, 0u, stage + T::kZ + L.wave * 256u);
+    }
 }
 
 // a_rd, b_rd: the lane's read addresses of step 0's activations (slice 0) and
 // of its weights in stage 0; tile: the weight tile of slot 0 (HALF: 1 on the
 // waves that run the up rows).
-template <int G, bool SYM, int NT, bool HALF>
+template <int G, bool SYM, int NT, bool HALF, int MODE>
 __device__ __forceinline__ void thin_kloop(const GemmLane<NT>& L, uint8_t* smem, uint32_t a_rd,
                                            uint32_t b_rd, uint32_t tile, f16v_t (&acc)[NT][2]) {
-    using T = ThinLds<SYM, NT>;
+    using T = ThinLds<SYM, NT, MODE>;
     constexpr uint32_t kLoads = (uint32_t)NT + (SYM ? 3u : 4u);
     const uint32_t last = L.nchunks - 1u;
+    if constexpr (T::kWindows) {
+#pragma unroll
+        for (uint32_t q = 0; q < 3u; ++q) thin_window<G, SYM, NT, MODE>(L, smem + T::kW, q, 0u);
+    }
     // chunks past the last repeat it: every chunk issues the same loads
 #pragma unroll
     for (uint32_t q = 0; q < T::kStages - 1u; ++q)
-        thin_issue<G, SYM, NT>(L, smem + q * T::kStage, q < last ? q : last);
+        thin_issue<G, SYM, NT, MODE>(L, smem, smem + q * T::kStage, q < last ? q : last);
     const uint32_t m = threadIdx.x & 31u, h = (threadIdx.x >> 5) & 1u;
-    const uint32_t s_rd = lds_addr(smem) + T::kS + L.wave * 256u + (32u * tile + m) * 4u;
+    // windows: the lane's row's 16 bytes in buffer 0; G = 32, half h reads group
+    // 2 c + h, the second half of the chunk's dword; G = 64, the groups of a row
+    // that starts off a dword lie one half word on
+    const uint32_t s_rd = lds_addr(smem) + (T::kWindows
+                              ? T::kW + L.wave * kGemmSWave + (32u * tile + m) * 16u
+                              : T::kS + L.wave * 256u + (32u * tile + m) * 4u);
+    const uint32_t sw0 = s_rd + (G == 32 ? 2u * h : L.s_own[0] & 2u);
+    const uint32_t sw1 = s_rd + 512u + (G == 32 ? 2u * h : L.s_own[1] & 2u);
+    const uint32_t zw0 = s_rd + T::kBufs * kGemmSBuf + (G == 32 ? 2u * h : L.z_own[0] & 2u);
+    const uint32_t zw1 = s_rd + T::kBufs * kGemmSBuf + 512u + (G == 32 ? 2u * h : L.z_own[1] & 2u);
+    uint32_t win = 0u;  // chunk c's buffer and its groups there
     uint32_t read = 0u, write = (T::kStages - 1u) * T::kStage;  // stages of chunk c and the one issued
 #pragma unroll 1
     for (uint32_t c = 0; c < L.nchunks; ++c) {
         wait_vmcnt<(T::kStages - 2u) * kLoads>();
         block_barrier();
         const uint32_t ahead = c + T::kStages - 1u;
-        thin_issue<G, SYM, NT>(L, smem + write, ahead < last ? ahead : last);
+        thin_issue<G, SYM, NT, MODE>(L, smem, smem + write, ahead < last ? ahead : last);
         u32x4_t af[2][NT], bw0, bw1;
         const uint32_t a = a_rd + read, b = b_rd + read;
         lds_read_act<NT, 0u>(af[0], a);
         bw0 = lds_read16<0>(b);
         bw1 = HALF ? bw0 : lds_read16<kGemmBTile>(b);
-        // G = 32: half h takes the dword's group 2 c + h; G = 64: the half
-        // that the row's alignment puts the group in
-        const uint32_t sh0 = G == 32 ? 2u * h : (L.s_own[0] + 2u * c) & 2u;
-        const uint32_t sh1 = G == 32 ? 2u * h : (L.s_own[1] + 2u * c) & 2u;
-        uint32_t s0 = lds_read_u16(s_rd + read + sh0);
-        uint32_t s1 = HALF ? s0 : lds_read_u16(s_rd + read + 128u + sh1);
-        uint32_t z0 = 0u, z1 = 0u;
-        if constexpr (!SYM) {
-            const uint32_t zh0 = G == 32 ? 2u * h : (L.z_own[0] + 2u * c) & 2u;
-            const uint32_t zh1 = G == 32 ? 2u * h : (L.z_own[1] + 2u * c) & 2u;
-            z0 = lds_read_u16(s_rd + read + (T::kZ - T::kS) + zh0);
-            z1 = HALF ? z0 : lds_read_u16(s_rd + read + (T::kZ - T::kS) + 128u + zh1);
+        uint32_t s0, s1, z0 = 0u, z1 = 0u;
+        if constexpr (T::kWindows) {
+            s0 = lds_read_u16(sw0 + win);
+            s1 = HALF ? s0 : lds_read_u16(sw1 + win);
+            if constexpr (!SYM) {
+                z0 = lds_read_u16(zw0 + win);
+                z1 = HALF ? z0 : lds_read_u16(zw1 + win);
+            }
+            constexpr uint32_t kStep = G == 32 ? 4u : 2u;
+            win += (c & 3u) != 3u ? kStep : kGemmSBuf - 3u * kStep;
+            if (win == T::kBufs * kGemmSBuf) win = 0u;
+        } else {
+            // G = 32: half h takes the dword's group 2 c + h; G = 64: the half
+            // that the row's alignment puts the group in
+            const uint32_t sh0 = G == 32 ? 2u * h : (L.s_own[0] + 2u * c) & 2u;
+            const uint32_t sh1 = G == 32 ? 2u * h : (L.s_own[1] + 2u * c) & 2u;
+            s0 = lds_read_u16(s_rd + read + sh0);
+            s1 = HALF ? s0 : lds_read_u16(s_rd + read + 128u + sh1);
+            if constexpr (!SYM) {
+                const uint32_t zh0 = G == 32 ? 2u * h : (L.z_own[0] + 2u * c) & 2u;
+                const uint32_t zh1 = G == 32 ? 2u * h : (L.z_own[1] + 2u * c) & 2u;
+                z0 = lds_read_u16(s_rd + read + (T::kZ - T::kS) + zh0);
+                z1 = HALF ? z0 : lds_read_u16(s_rd + read + (T::kZ - T::kS) + 128u + zh1);
+            }
         }
         lds_wait<NT>(af[0], bw0, bw1, s0, s1, z0, z1);
         const GroupScale g0 = group_scale<SYM>((uint16_t)s0, (uint16_t)z0);
@@ -731,7 +791,7 @@ __device__ __forceinline__ void gemm_block(const GemmArgs& args, const tsg_route
     }
     if constexpr (THIN) {
         const uint32_t up = MODE == 0 && HALF && L.wave >= 2u ? 1u : 0u;
-        thin_kloop<G, SYM, NT, HALF>(L, smem, L.a_rd, L.b_rd - Y::kBBase + ThinLds<SYM, NT>::kB, up, acc);
+        thin_kloop<G, SYM, NT, HALF, MODE>(L, smem, L.a_rd, L.b_rd - Y::kBBase + NT * 4096u, up, acc);
     } else {
         gemm_kloop<R, G, SYM, NT, HALF>(L, smem, acc);
     }
@@ -966,16 +1026,19 @@ __device__ __forceinline__ void gemm_item(const GemmArgs& args, const tsg_routed
 // The routed GEMMs of a call whose experts have few rows each, in passes of
 // kThinRows rows. Such a call is bound by latency: a weight is dequantised for
 // one or two MFMAs, so a chunk is barrier, LDS reads, dequantisation and MFMAs
-// in turn (0.5 us alone), and two workgroups per CU, which is what the wide
-// kernels' accumulators and rings allow, hide little of it. With a third of
-// the LDS and at most 168 registers three fit. Gate/up and down of 67 tokens,
-// 8 of 128 experts, 2816 x 704: 126 us in the fused launch, 99 here (104 with
-// two per CU and deeper rings, 100 with four and shallower ones; 121 with
-// passes of 32 rows); of 32 tokens 102 and 83; of 9 tokens 86 and 51. Grid:
-// x = items as in moe_gemm_kernel, y = the passes side by side.
+// in turn (0.5 us alone); deeper rings and, in down, three workgroups per CU
+// (the wide kernels' accumulators and rings allow two) hide more of it. Gate/up
+// and down of 67 tokens, 8 of 128 experts, 2816 x 704, sym g32, four layers in
+// turn, fused launch and here: logits with half their variance in common (67
+// experts) 131 and 93 us, with none (126 experts) 158 and 158; 9 tokens 94 and
+// 54, 125 and 96. With a dword of scales a row and chunk in gate/up too and
+// three workgroups per CU they were 104, 182, 56 and 105, and affine g32, which
+// reads twice the parameters, 134 and 274 for 67 tokens (107 and 192 here, 148
+// and 199 fused). Grid: x = items as in moe_gemm_kernel, y = the passes side
+// by side.
 template <int G, bool SYM, int ACT, int MODE>
-__global__ __launch_bounds__(kGemmThreads, 3) void moe_gemm_thin_kernel(GemmArgs args) {
-    extern __shared__ __align__(16) uint8_t smem[];  // kThinLds
+__global__ __launch_bounds__(kGemmThreads, thin_per_cu(MODE)) void moe_gemm_thin_kernel(GemmArgs args) {
+    extern __shared__ __align__(16) uint8_t smem[];  // ThinLds::kBytes
     const uint32_t nb = args.n_blocks_device ? min(*args.n_blocks_device, args.n_blocks) : args.n_blocks;
     if (blockIdx.x >= nb * args.ntiles) return;
     uint32_t yb, tile;
@@ -1133,16 +1196,23 @@ __global__ __launch_bounds__(kGemmThreads, 2) void moe_gemm_fused_kernel(GemmArg
 
 // Whether a device-written work list goes to the thin kernels. The host knows
 // of it only its capacity: of tsg_prefill_group_pairs_device's ceil(pairs /
-// 128) + E entries, those past E count the pairs. 16 are 2048 pairs: gate/up
-// and down of 256 tokens, 2816 x 704, 128 experts, are 192 us fused and 182
-// thin, of 400 tokens 197 and 225 (256 experts of 2048 x 512: 141 and 127, 153
-// and 176 at 509; 32 experts: 115 and 97 at 300). The affine kernels read the
-// zero points too and hold 150 registers: 67 tokens are 135 and 109, 128
-// tokens 162 and 171, so their line is 6, 768 pairs. With three workgroups per
-// CU, each on part of 256 weight rows' lines, wider experts outgrow the L2:
-// 40 tokens of 2048 x 1024 are 124 and 98, of 4096 x 1536 237 and 253 (affine
-// 271 and 361), so d * f stays at 2^21 (2816 x 704 is 1.98 M). A list with
-// spare capacity goes to the wide kernels, with the same results.
+// tile_rows) + E entries, those past E count the pairs. 16 are 2048 pairs in
+// blocks of 128 rows, 4096 of 256, 1024 of 64. Fused launch and thin kernels,
+// us, 2816 x 704 of 128 experts, sym g32, logits with half their variance in
+// common and (in brackets) with none, the routing that reads most experts:
+// 2048 pairs 189 and 144 (159 and 155), 3072 196 and 169 (166 and 167), 4096
+// 199 and 181 (178 and 179), in blocks of 256 rows 280 and 210 (178 and 177);
+// 256 experts of 2048 x 512 131 and 102 (155 and 151) at 2048, in blocks of 256
+// 247 and 144 (158 and 155) at 4096. Few experts gain too (8 experts, 2048
+// pairs: 87 and 59). The worst met is 536 pairs evenly over 256 experts of 2048
+// x 512, 132 and 137. Affine lists stop at 6, 768 pairs of 128 rows (g64 150 and 104, 170
+// and 171 in brackets; g32 172 and 122, 201 and 197): at 2048 they would gain
+// too (189 and 150, 171 and 165) and are left as they were. Wider experts: 40
+// tokens over 64 experts of 2048 x 1024 are 108 and 71 (109 and 87), affine g32
+// 111 and 78; of 4096 x 1536 209 and 180 (234 and 229), affine 252 and 249 (302
+// and 307) and, 96 tokens, 285 and 313, so d * f stays at 2^21 (2816 x 704 is
+// 1.98 M). A list with spare capacity goes to the wide kernels, with the same
+// results.
 template <bool SYM>
 inline bool few_rows(const GemmArgs& a, uint32_t max_blocks) {
     return a.n_blocks_device && max_blocks <= (uint64_t)a.num_experts + (SYM ? 16u : 6u) &&
@@ -1153,10 +1223,14 @@ template <int G, bool SYM, int MODE>
 tsg_status launch_thin(const tsg_moe* moe, hipStream_t s, const GemmArgs& args, uint32_t max_blocks) {
     auto kern = moe->activation == TSG_ACT_SILU ? moe_gemm_thin_kernel<G, SYM, TSG_ACT_SILU, MODE>
                                                 : moe_gemm_thin_kernel<G, SYM, TSG_ACT_GELU_TANH, MODE>;
-    // blocks of up to two passes (what the device grouping writes at most)
-    // run them side by side
+    // the passes of a block of 128 rows run side by side; those of wider blocks
+    // (256 rows: four) two by two
     const dim3 grid(args.ntiles * max_blocks, 2u);
-    hipLaunchKernelGGL(kern, grid, dim3(kGemmThreads), kThinLds, s, args);
+    constexpr uint32_t lds = ThinLds<SYM, 1, MODE>::kBytes;
+    if (lds > 64u * 1024u)
+        TSG_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(kern, grid, dim3(kGemmThreads), lds, s, args);
     return check_launch(MODE == 0 ? "moe_gemm thin gate/up" : "moe_gemm thin down");
 }
 
