@@ -197,8 +197,9 @@ def test_shared_expert_int4_matches_steps_and_oracle(tsg, ctx, d, f, group, symm
                                                  (128, 4160, 32, True), (4160, 992, 32, False)])
 def test_shared_expert_int4_scratch_and_shared_buffers(tsg, ctx, d, f, group, symmetric):
     """At small and large f and at d past one batch of chunks: the scratch
-    holds the halves and the activation the separate calls leave there, and the
-    activation may share a buffer with a half or with x."""
+    holds the halves and the activation the separate calls leave there; the
+    activation may share a buffer with a half or with x, and the halves one
+    with each other, as in those calls."""
     configure(ctx, group, symmetric)
     S, q = tsg.SharedExpertInt4(ctx), tsg.DequantInt4GEMV(ctx)
     gate, up, down, x = _dense_parts(d, f, group, 0x71 + f, symmetric)
@@ -220,6 +221,19 @@ def test_shared_expert_int4_scratch_and_shared_buffers(tsg, ctx, d, f, group, sy
         y.fill_(0)
         S.encode(dev(x), *proj, y, g, u, a)
         assert np.array_equal(host(y, np.uint16), want)
+    # both halves in one buffer, and the up half's start in the gate half's end:
+    # the calls one after the other, whose activation reads what the up
+    # projection left of the gate half
+    for shift in (0, 32):
+        halves = empty(f + shift)
+        q.encode(dv[0][0], dv[0][1], bias(dv[0]), dev(x), halves[:f], f, d)
+        q.encode(dv[1][0], dv[1][1], bias(dv[1]), dev(x), halves[shift:], f, d)
+        S.encode_gelu_mul(halves[:f], halves[shift:], a1, f)
+        q.encode(dv[2][0], dv[2][1], bias(dv[2]), a1, y1, d, f)
+        mixed = empty(f + shift)
+        S.encode(dev(x), *proj, y, mixed[:f], mixed[shift:], sa)
+        for got, ref in ((mixed, halves), (sa, a1), (y, y1)):
+            assert np.array_equal(host(got, np.uint16), host(ref, np.uint16)), shift
     both = empty(max(d, f))  # x and the activation in one buffer
     both[:d] = dev(x)
     y.fill_(0)

@@ -363,10 +363,24 @@ extern "C" tsg_status tsg_shared_expert_int4(
                         up->cols)))
         return st;
     TSG_REQUIRE(scratch_act, TSG_ERR_INVALID_ARGUMENT, "NULL operand");
-    // the activation may lie in x's buffer (x is not needed after the
-    // projections), which one launch would overwrite while it is still read
-    const uintptr_t xa = reinterpret_cast<uintptr_t>(x), aa = reinterpret_cast<uintptr_t>(scratch_act);
-    if (aa < xa + gate->cols * 2ull && xa < aa + required) {
+    // One launch needs x and the halves apart, and the activation apart from x
+    // and from each half or in its place. Where buffers share bytes otherwise
+    // (the activation in x's buffer, both halves in one) the separate launches
+    // keep their order of reads and writes.
+    const uint64_t x_len = (uint64_t)gate->cols * 2u;
+    auto apart = [](const uint16_t* a, uint64_t an, const uint16_t* b, uint64_t bn) {
+        const uintptr_t a0 = reinterpret_cast<uintptr_t>(a), b0 = reinterpret_cast<uintptr_t>(b);
+        return a0 + an <= b0 || b0 + bn <= a0;
+    };
+    auto in_place = [&](const uint16_t* half) {
+        return scratch_act == half || apart(scratch_act, required, half, required);
+    };
+    const bool one_launch = apart(x, x_len, scratch_act, required) &&
+                            apart(x, x_len, scratch_gate, required) &&
+                            apart(x, x_len, scratch_up, required) &&
+                            apart(scratch_gate, required, scratch_up, required) &&
+                            in_place(scratch_gate) && in_place(scratch_up);
+    if (!one_launch) {
         if ((st = tsg_qmv_int4(ctx, stream, gate->weights, gate->scales, gate->biases, x,
                                scratch_gate, gate->rows, gate->cols)) ||
             (st = tsg_qmv_int4(ctx, stream, up->weights, up->scales, up->biases, x, scratch_up,
