@@ -527,6 +527,38 @@ def test_few_rows_gemms_equal_the_wide_ones(tsg, ctx, group, scheme, act, d, f):
         assert np.array_equal(a, out[0][0]) and np.array_equal(p, out[0][1])
 
 
+@pytest.mark.parametrize("capacity", [12, 21])
+def test_grouped_gemms_stay_inside_the_list(tsg, ctx, capacity):
+    """A device count above the list's capacity: the grouped GEMMs (few-rows
+    kernels at 12 blocks of 2 experts, the wide ones at 21) run the capacity's
+    blocks and nothing behind them. The buffers hold all 40 blocks."""
+    configure(ctx, 32, "sym")
+    ne, d, f, blocks, rows = 2, 256, 192, 40, 3
+    t = blocks * rows
+    rng = oracle.SplitMix64(0x11F7)
+    parts = [[oracle.quantize_int4(rng.uniforms(-0.125, 0.125, r * c).reshape(r, c), 32, True)
+              for r, c in ((f, d), (f, d), (d, f))] for _ in range(ne)]
+    layer = _upload_layer(tsg, ctx, parts, True)[0]
+    pairs = np.zeros(t, oracle.PAIR_DTYPE)
+    pairs["token"] = np.arange(t)
+    listed = np.array([(b % ne, rows * b, rows, rows * b) for b in range(blocks)], oracle.BLOCK_DTYPE)
+    hidden, P, B = dev(rng.uniforms_f16(-1, 1, t * d)), dev(pairs), dev(listed)
+    nb = dev(np.array([blocks], np.uint32))
+    g = tsg.PrefillGroupedRoutedMoE(tsg.MoE(ctx))
+    for fused in (False, True):
+        act, part = empty(t * f, fill=NAN16), empty(t * d, fill=NAN16)
+        if fused:
+            g.encode_gate_up_down(layer, hidden, d, P, B, capacity, act, part, 1, d, f,
+                                  n_blocks_device=nb)
+        else:
+            g.encode_gate_up(layer, hidden, d, P, B, capacity, act, d, f, n_blocks_device=nb)
+            g.encode_down(layer, act, P, B, capacity, part, 1, d, f, n_blocks_device=nb)
+        ctx.synchronize()
+        for buf, width in ((act, f), (part, d)):
+            written = ~np.isnan(host(buf, np.uint16).view(np.float16).reshape(t, width)).any(axis=1)
+            assert np.array_equal(written, np.arange(t) < rows * capacity), fused
+
+
 @pytest.mark.parametrize("ne,d,f,pairs,group,scheme", [(128, 2816, 704, 768, 32, "affine"),
                                                        (256, 2048, 512, 536, 32, "affine"),
                                                        (256, 2048, 512, 1024, 32, "sym")])

@@ -1073,7 +1073,7 @@ template <int G, bool SYM, int ACT, int MODE>
 __global__ __launch_bounds__(kGemmThreads, 2) void moe_gemm_kernel(GemmArgs args) {
     extern __shared__ __align__(16) uint8_t smem[];  // GemmLds<gemm_rows<MODE>()>::bytes(SYM)
     constexpr uint32_t R = gemm_rows<MODE>();
-    const uint32_t nb = args.n_blocks_device ? *args.n_blocks_device : args.n_blocks;
+    const uint32_t nb = args.n_blocks_device ? min(*args.n_blocks_device, args.n_blocks) : args.n_blocks;
     const uint32_t total = nb * args.ntiles;
     if (blockIdx.x >= total) return;
     uint32_t yb, tile;
