@@ -523,14 +523,15 @@ def run_fused_vs_two_launches(tsg, ctx, layer, t, d, f, ne, s, act, seed, tile=2
                               device_list=True):
     """tsg_prefill_moe_gate_up_down against tsg_prefill_moe_gate_up then
     tsg_prefill_moe_down on the same grouping: act and route partials equal
-    bit for bit."""
+    bit for bit. A device list has 40 entries to spare: a tight one of few
+    pairs would take the few-rows kernels in place of the fused launch."""
     k = 8
     rng = np.random.default_rng(seed)
     idx, w = wl.zipf_routing(rng, t, ne, k, s)
     hidden = dev(wl.f16_normal(rng, t * d))
     moe = tsg.MoE(ctx, gate_activation=act)
     g = tsg.PrefillGroupedRoutedMoE(moe)
-    max_blocks = -(-t * k // tile) + ne
+    max_blocks = -(-t * k // tile) + ne + 40
     sp, off, cnt = empty(t * k * 4, np.uint32), empty(ne, np.uint32), empty(ne, np.uint32)
     blocks, nb = empty(max_blocks * 4, np.uint32), empty(1, np.uint32)
     scratch = empty(g.scratch_bytes(t, k, ne) // 4 + 1, np.uint32)
@@ -596,11 +597,13 @@ def test_fused_gate_up_down_rejects_unaligned_act(tsg, ctx, gemma_layer):
     ctx.synchronize()
 
 
-def test_grouped_gemm_skips_and_reports_expert_past_layer(tsg, ctx, gemma_layer):
+@pytest.mark.parametrize("device_capacity", [0, 2, 200])
+def test_grouped_gemm_skips_and_reports_expert_past_layer(tsg, ctx, gemma_layer, device_capacity):
     """A block list written on the device is not seen by the host: a block
     naming an expert past the layer is skipped by the grouped GEMM (two-launch
-    and fused forms) and tsg_ctx_synchronize reports it; the other blocks'
-    rows are written as usual."""
+    and one-call forms) and tsg_ctx_synchronize reports it; the other blocks'
+    rows are written as usual. The list is host-counted (0), or device-counted
+    with a capacity of the few-rows kernels (2) or of the wide ones (200)."""
     configure(ctx, 32, "sym")
     layer = gemma_layer[0]
     d, f, k, t = 2816, 704, 8, 4
@@ -608,30 +611,37 @@ def test_grouped_gemm_skips_and_reports_expert_past_layer(tsg, ctx, gemma_layer)
     pairs = np.zeros(t * k, oracle.PAIR_DTYPE)
     pairs["token"] = np.repeat(np.arange(t, dtype=np.uint32), k)
     pairs["rank"] = np.tile(np.arange(k, dtype=np.uint32), t)
-    blocks = np.array([(3, 0, 16, 0), (500, 16, 16, 16)], dtype=oracle.BLOCK_DTYPE)
+    blocks = np.zeros(max(2, device_capacity), oracle.BLOCK_DTYPE)
+    blocks[:2] = [(3, 0, 16, 0), (500, 16, 16, 16)]
     hidden = dev(wl.f16_normal(np.random.default_rng(5), t * d))
     P, B = dev(pairs), dev(blocks.view(np.uint32))
+    n = device_capacity or 2
+    kw = dict(n_blocks_device=dev(np.array([2], np.uint32))) if device_capacity else {}
     for fused in (False, True):
         act, part = empty(t * k * f, fill=NAN16), empty(t * k * d, fill=NAN16)
         if fused:
-            g.encode_gate_up_down(layer, hidden, d, P, B, 2, act, part, k, d, f)
+            g.encode_gate_up_down(layer, hidden, d, P, B, n, act, part, k, d, f, **kw)
         else:
-            g.encode_gate_up(layer, hidden, d, P, B, 2, act, d, f)
-            g.encode_down(layer, act, P, B, 2, part, k, d, f)
+            g.encode_gate_up(layer, hidden, d, P, B, n, act, d, f, **kw)
+            g.encode_down(layer, act, P, B, n, part, k, d, f, **kw)
         with pytest.raises(tsg.TsgError) as e:
             ctx.synchronize()
         assert "past the layer" in str(e.value)
         a = host(act, np.uint16).reshape(t * k, f)
         assert np.all(np.isfinite(oracle.f16_to_float(a[:16]))), "the valid block's rows"
         assert np.all(a[16:] == NAN16), "the skipped block wrote nothing"
+        p = host(part, np.uint16).reshape(t * k, d)
+        assert np.all(np.isfinite(oracle.f16_to_float(p[:16]))) and np.all(p[16:] == NAN16)
     ctx.synchronize()  # the error word was cleared
 
 
-def test_fused_gate_up_down_zero_row_blocks(tsg, ctx, gemma_layer):
+@pytest.mark.parametrize("few_rows", [False, True])
+def test_fused_gate_up_down_zero_row_blocks(tsg, ctx, gemma_layer, few_rows):
     """Routed blocks with no rows, between real ones, are no-ops in both
     forms: the fused launch (64 blocks, 1,088 items, so every workgroup takes
     several and meets zero-row items after others) equals the two launches
-    bit for bit and drains its schedule, twice in a row."""
+    bit for bit and drains its schedule, twice in a row; so do the few-rows
+    kernels, which a device-counted list of that capacity takes."""
     configure(ctx, 32, "sym")
     layer = gemma_layer[0]
     d, f, k, t = 2816, 704, 8, 64
@@ -653,18 +663,21 @@ def test_fused_gate_up_down_zero_row_blocks(tsg, ctx, gemma_layer):
     g.encode_down(layer, a2, P, B, 64, p2, k, d, f)
     want_a, want_p = host(a2, np.uint16), host(p2, np.uint16)
     assert np.all(np.isfinite(oracle.f16_to_float(want_p)))
+    count = dev(np.array([64], np.uint32)) if few_rows else None
     for rep in range(2):
         a1, p1 = empty(t * k * f, fill=NAN16), empty(t * k * d, fill=NAN16)
-        g.encode_gate_up_down(layer, hidden, d, P, B, 64, a1, p1, k, d, f)
+        g.encode_gate_up_down(layer, hidden, d, P, B, 64, a1, p1, k, d, f, n_blocks_device=count)
         ctx.synchronize()
         assert np.array_equal(host(a1, np.uint16), want_a), f"act differs (launch {rep})"
         assert np.array_equal(host(p1, np.uint16), want_p), f"partials differ (launch {rep})"
 
 
-def test_fused_gate_up_down_empty_device_list(tsg, ctx, gemma_layer):
-    """A device count of zero (no routed block) runs the fused launch to its
-    end without work, writes nothing and reports nothing; the next launch on
-    the same context still runs a real list (the schedule was left reset)."""
+@pytest.mark.parametrize("capacity", [1, 200])
+def test_fused_gate_up_down_empty_device_list(tsg, ctx, gemma_layer, capacity):
+    """A device count of zero (no routed block) runs the fused launch (capacity
+    200; the few-rows kernels at 1) to its end without work, writes nothing and
+    reports nothing; the next launch on the same context still runs a real
+    list (the schedule was left reset)."""
     configure(ctx, 32, "sym")
     layer = gemma_layer[0]
     d, f, k, t = 2816, 704, 8, 4
@@ -672,18 +685,19 @@ def test_fused_gate_up_down_empty_device_list(tsg, ctx, gemma_layer):
     pairs = np.zeros(t * k, oracle.PAIR_DTYPE)
     pairs["token"] = np.repeat(np.arange(t, dtype=np.uint32), k)
     pairs["rank"] = np.tile(np.arange(k, dtype=np.uint32), t)
-    blocks = np.array([(3, 0, t * k, 0)], dtype=oracle.BLOCK_DTYPE)
+    blocks = np.zeros(capacity, oracle.BLOCK_DTYPE)
+    blocks[0] = (3, 0, t * k, 0)
     hidden = dev(wl.f16_normal(np.random.default_rng(9), t * d))
     P, B = dev(pairs), dev(blocks.view(np.uint32))
     act, part = empty(t * k * f, fill=NAN16), empty(t * k * d, fill=NAN16)
-    g.encode_gate_up_down(layer, hidden, d, P, B, 1, act, part, k, d, f,
+    g.encode_gate_up_down(layer, hidden, d, P, B, capacity, act, part, k, d, f,
                           n_blocks_device=dev(np.zeros(1, np.uint32)))
     ctx.synchronize()
     assert np.all(host(act, np.uint16) == NAN16) and np.all(host(part, np.uint16) == NAN16)
     a2, p2 = empty(t * k * f, fill=NAN16), empty(t * k * d, fill=NAN16)
     g.encode_gate_up(layer, hidden, d, P, B, 1, a2, d, f)
     g.encode_down(layer, a2, P, B, 1, p2, k, d, f)
-    g.encode_gate_up_down(layer, hidden, d, P, B, 1, act, part, k, d, f,
+    g.encode_gate_up_down(layer, hidden, d, P, B, capacity, act, part, k, d, f,
                           n_blocks_device=dev(np.ones(1, np.uint32)))
     ctx.synchronize()
     assert np.array_equal(host(act, np.uint16), host(a2, np.uint16))
