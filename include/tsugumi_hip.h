@@ -670,9 +670,13 @@ tsg_status tsg_prefill_moe_reduce_token_major(tsg_ctx* ctx, tsg_stream stream,
  * W is [n, k/2] bytes, scales and biases [n, k/group] bf16 (biases unused
  * under sym). The dequant-to-LDS MFMA GEMM of the routed experts, rows taken
  * in order; few workgroups' worth of rows and columns split K over waves
- * instead (fp32 partial sums, a fixed order for a given t, n and k). Errors: K % group != 0 (the reference's precondition). Declined
- * with TSG_ERR_UNSUPPORTED: K or N not a multiple of 64, t*n or t*k >= 2^32,
- * or W of 4 GiB or more. */
+ * instead. Both sum in fp32 and in an order that is fixed for the call, but not
+ * in the same one: t, n, k, the device's count of compute units and whether y
+ * and x share bytes choose between them, so a row's last bits can differ
+ * between calls of other row counts. y may overlap x only where one column
+ * tile holds all of a row (n up to 128). Errors: K % group != 0 (the
+ * reference's precondition). Declined with TSG_ERR_UNSUPPORTED: K or N not a
+ * multiple of 64, t*n or t*k >= 2^32, or W of 4 GiB or more. */
 tsg_status tsg_prefill_int4_qmm(tsg_ctx* ctx, tsg_stream stream, const uint8_t* weights,
                                 const uint16_t* scales, const uint16_t* biases,
                                 const uint16_t* x, uint16_t* y, uint32_t t, uint32_t n,

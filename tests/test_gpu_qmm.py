@@ -140,6 +140,12 @@ def test_qmm_of_few_rows(tsg, t, n, k, g, scheme):
     of each result (2^-11 of it) and K fp32 roundings (K 2^-24 of the sum of
     the magnitudes). The rows past y keep their bytes."""
     print(f"qmm few rows t={t} n={n} k={k} g{g} {scheme}", flush=True)
+    check_elements(tsg, t, n, k, g, scheme)
+
+
+def check_elements(tsg, t, n, k, g, scheme, in_place=False):
+    """Every element against fp64, in the bound of test_qmm_of_few_rows; y past
+    t rows keeps its bytes. in_place: y is x's buffer (n == k)."""
     sym = scheme == "sym"
     ctx = tsg.Context(0, group_size=g)
     ctx.set_affine_scheme(scheme)
@@ -147,8 +153,11 @@ def test_qmm_of_few_rows(tsg, t, n, k, g, scheme):
     packed, scales, biases = operands(rng, n, k, g)
     xb = oracle.f16_bits(rng.normal(0, 1, t * k).astype(np.float32))
     y = empty(t * n + 64, fill=0x1234)
+    x_dev = y if in_place else dev(xb)
+    if in_place:
+        y[:t * k] = dev(xb)
     tsg.PrefillInt4QMM(ctx).encode(dev(packed), dev(scales), None if sym else dev(biases),
-                                   dev(xb), y, t, n, k)
+                                   x_dev, y, t, n, k)
     got = host(y, np.uint16)
     assert np.all(got[t * n:] == 0x1234)
     s = np.repeat(oracle.bf16_to_float(scales).reshape(n, k // g).astype(np.float32), g, axis=1)
@@ -162,3 +171,24 @@ def test_qmm_of_few_rows(tsg, t, n, k, g, scheme):
     err = np.abs(oracle.f16_to_float(got[:t * n]).reshape(t, n) - ref)
     assert np.all(err <= np.abs(ref) * 2.0 ** -11 + mag * k * 2.0 ** -24 + 2.0 ** -25)
     ctx.close()
+
+
+@pytest.mark.parametrize("g,scheme", [(32, "sym"), (64, "affine")])
+@pytest.mark.parametrize("t,n,k", [(1025, 2880, 704), (1100, 2880, 2816), (1100, 2880, 704),
+                                   (2049, 4160, 704), (2112, 4160, 704)])
+def test_qmm_gemm_at_ragged_tiles(tsg, t, n, k, g, scheme):
+    """The GEMM at row blocks of 1, 64 and 76 rows past full ones (one, two and
+    three slices) and at a last column tile of 64 live columns: 128-column tiles
+    (n = 2880) and 256-column ones, three of whose waves are dead (n = 4160 from
+    2049 rows), per element."""
+    print(f"qmm gemm ragged t={t} n={n} k={k} g{g} {scheme}", flush=True)
+    check_elements(tsg, t, n, k, g, scheme)
+
+
+@pytest.mark.parametrize("t,n", [(100, 128), (200, 64)])
+def test_qmm_in_place(tsg, t, n):
+    """y in x's buffer where one column tile holds all columns: each row block
+    has read its rows when it writes them. Few rows as these go to the K split
+    otherwise, whose workgroups would read rows that others have written."""
+    print(f"qmm in place t={t} n={n}", flush=True)
+    check_elements(tsg, t, n, n, 32, "sym", in_place=True)
