@@ -192,3 +192,30 @@ def test_qmm_in_place(tsg, t, n):
     otherwise, whose workgroups would read rows that others have written."""
     print(f"qmm in place t={t} n={n}", flush=True)
     check_elements(tsg, t, n, n, 32, "sym", in_place=True)
+
+
+@pytest.mark.parametrize("t,n,k,g,scheme", [
+    (32, 704, 512, 32, "sym"), (130, 704, 512, 32, "affine"), (32, 2048, 384, 64, "affine"),
+    (25, 704, 256, 32, "sym"), (40, 2048, 448, 64, "affine"), (32, 8256, 2560, 32, "affine"),
+    (25, 16384, 2112, 32, "sym"), (64, 4160, 3584, 32, "sym"), (36, 8192, 2560, 32, "affine"),
+    (96, 5440, 3584, 32, "affine"), (64, 8192, 4096, 64, "affine"),
+])
+def test_qmm_rows_past_the_split_keep_the_gemms_bits(tsg, t, n, k, g, scheme):
+    """Few rows that the K split once took although the GEMM is the faster:
+    their rows are those of a call of 2048 rows, bit for bit (the GEMM's sum does
+    not depend on the rows beside a row)."""
+    print(f"qmm past the split t={t} n={n} k={k} g{g} {scheme}", flush=True)
+    import torch
+    sym = scheme == "sym"
+    ctx = tsg.Context(0, group_size=g)
+    ctx.set_affine_scheme(scheme)
+    rng = np.random.default_rng(t + n + k)
+    packed, scales, biases = operands(rng, n, k, g)
+    x = dev(oracle.f16_bits(rng.normal(0, 1, 2048 * k).astype(np.float32)))
+    W, S, B = dev(packed), dev(scales), None if sym else dev(biases)
+    few, many = empty(t * n), empty(2048 * n)
+    q = tsg.PrefillInt4QMM(ctx)
+    q.encode(W, S, B, x, few, t, n, k)
+    q.encode(W, S, B, x, many, 2048, n, k)
+    assert torch.equal(few, many[:t * n])
+    ctx.close()

@@ -1279,16 +1279,14 @@ tsg_status launch_fused(const tsg_moe* moe, hipStream_t s, GemmArgs gu, GemmArgs
     return check_launch("moe_gemm fused gate/up + down");
 }
 
-// Dense projection: blocks of kDenseRows (128) rows of x in order, 256
-// output columns per workgroup (the down GEMM's tiling).
 // The dense projection of few rows: 32 rows x 32 weight rows a workgroup, the
 // chunks of K dealt to its kSplitWaves waves, whose fp32 accumulators are
 // added in wave order through LDS. With 128 columns a workgroup, 67 rows x 4096
 // columns are 32 workgroups on 256 CUs, each a chain of K / 64 chunks of
 // 0.5 us; here they are 384 with an eighth of the chain and no barrier in it,
 // the operands in registers three chunks ahead. Bound by the L1: a lane reads
-// its own row, so a load touches 32 lines. K = 2816: 67 x 4096 24.9 -> 17.2 us,
-// 9 rows 20.5 -> 7.9, 704 columns of 256 rows 29.5 -> 11.8.
+// its own row, so a load touches 32 lines. K = 2816: 67 x 4096 26.0 -> 17.4 us,
+// 9 rows 21.0 -> 8.3, 704 columns of 256 rows 29.9 -> 12.5.
 constexpr uint32_t kSplitWaves = 8;
 
 // One lane's operands of a chunk: K 64 c + 32 h .. + 32 of its activation row
@@ -1359,28 +1357,62 @@ __global__ __launch_bounds__(64u * kSplitWaves, 4) void qmm_split_kernel(GemmArg
 }
 static_assert(64u * kSplitWaves == 32u * 16u, "one thread per pair of outputs");
 
+// Where the K split is the faster of the two. Its time goes in steps of a
+// workgroup per CU, and a step's by the rows of its blocks (the rows past the
+// last repeat one, whose lines the L1 holds); the GEMM's hardly grows until its
+// own grid fills the device, but with the slices of a row block. us, GEMM and
+// split, sym g32 unless named:
+//  - one step: K = 2816, 9 rows x 4096 21.0 and 8.3, 32 rows 21.2 and 12.2, 64
+//    rows 23.4 and 12.6; K = 704, 256 x 1024 10.5 and 7.0. With K below 704 the
+//    split's fixed part is most of it: 32 rows x 2048 lose from K = 256 (affine
+//    g64 384: 5.4 and 6.0, 192: 5.2 and 4.9), affine 40 too (448: 5.7 and 6.1),
+//    24 and 96 rows gain. K = 512 loses nearly everywhere (32 x 8192 6.3 and
+//    8.4, 96 x 2688 7.8 and 8.4, 128 rows affine g32 9.0 and 9.5): rows an odd
+//    multiple of 1 KB apart meet in the L1, as those of K = 2560 and 3584 do
+//    (64 x 4160, us a chunk: 0.59 at 2560, 0.50 at 2816, 0.49 at 3072), and
+//    there it is a short K besides.
+//  - two steps: worth it for K past 2048 (2048 x 2048, 256 rows 23.4 both; 1024
+//    x 704, 320 rows 10.6 and 11.9) where the GEMM runs four slices (128 rows x
+//    4096 x 2816 30.3 and 22.5, affine g32 31.1 and 24.6, its closest 38.2 and
+//    36.5 at K = 3584) or the second step's blocks are not full: 67 rows x 4096
+//    x 2816 26.0 and 17.4, 40 x 8192 23.6 and 18.5, but 64 x 8192 x 3584 29.1
+//    and 32.0, 32 x 16384 x 3584 27.0 and 32.2 (affine g32, which reads twice
+//    the parameters, 28.1 and 36.7). The table has the most rows at which no K
+//    from 2112 to 8192 was slower by more than 4 %.
+//  - three steps nowhere (4096 x 2816, 160 rows: 29.9 and 30.8).
+template <int G, bool SYM>
+inline bool split_pays(uint32_t rows, uint32_t cols, uint32_t K, uint32_t num_cus) {
+    const uint32_t row_blocks = (rows + 31u) / 32u, col_tiles = cols / 32u;
+    const uint32_t slices = row_blocks < 4u ? row_blocks : 4u;
+    const uint64_t groups = (uint64_t)row_blocks * col_tiles;
+    if (K == 512u) return false;
+    if (groups <= num_cus) return K < 256u || K > 640u || (slices == 1u ? rows <= 24u : SYM || slices > 2u);
+    if (groups > 2u * num_cus || K <= 2048u) return false;
+    const bool last_block = (uint64_t)(row_blocks - 1u) * col_tiles <= num_cus;  // the second step runs only it
+    const uint32_t second = last_block ? rows - 32u * (row_blocks - 1u) : 32u;
+    const bool meet = K % 1024u == 512u;
+    constexpr uint32_t kMost[4][4] = {{24u, 32u, 32u, 32u},   // sym
+                                      {20u, 16u, 32u, 32u},   // sym of rows that meet; affine g64
+                                      {20u, 8u, 32u, 32u},    // affine g32
+                                      {12u, 0u, 16u, 32u}};   // affine g32 of rows that meet
+    return second <= kMost[SYM ? (meet ? 1 : 0) : G == 64 ? 1 : meet ? 3 : 2][slices - 1u];
+}
+
+// A y that overlaps x keeps the GEMM's order of reads and writes.
 template <int G, bool SYM>
 tsg_status launch_dense_qmm(hipStream_t s, const GemmArgs& a, uint32_t num_cus) {
     GemmArgs args = a;
-    // Few workgroups: the K split. Its time goes in steps of a workgroup per CU
-    // (11.5 us at K = 2816, 12.4 at 2048, 6.8 at 704), the GEMM's hardly grows
-    // until its own grid fills the device. One step is always the faster (2048 x
-    // 2048, 128 rows: 22.8 and 12.7; 1024 x 704, 256 rows: 10.8 and 7.1); two are
-    // where K is long (4096 x 2816, 128 rows: 29.8 and 21.6; 2816 x 4096: 41.0
-    // and 30.7; but 2048 x 2048, 256 rows: 23.0 and 23.3, affine 27.0; 1024 x
-    // 704, 320 rows: 10.8 and 11.9), three nowhere (4096 x 2816, 160 rows: 29.9
-    // and 30.8). A y that overlaps x keeps the GEMM's order of reads and writes.
-    const uint64_t split = (uint64_t)(a.d / 32u) * ((a.dense_rows + 31u) / 32u);
     const uintptr_t x0 = reinterpret_cast<uintptr_t>(a.a), y0 = reinterpret_cast<uintptr_t>(a.out);
     const bool apart = x0 + (uint64_t)a.dense_rows * a.f * 2u <= y0 ||
                        y0 + (uint64_t)a.dense_rows * a.d * 2u <= x0;
-    if (split <= (a.f > 2048u ? 2u : 1u) * num_cus && apart) {
+    if (apart && split_pays<G, SYM>(a.dense_rows, a.d, a.f, num_cus)) {
         hipLaunchKernelGGL((qmm_split_kernel<G, SYM>), dim3(a.d / 32u, (a.dense_rows + 31u) / 32u),
                            dim3(64u * kSplitWaves), 0, s, args);
         return check_launch("qmm split");
     }
+    // Otherwise the GEMM: blocks of kDenseRows (128) rows of x in order.
     args.n_blocks = (a.dense_rows + kDenseRows - 1u) / kDenseRows;
-    // 256-column tiles while they cover the device's CUs; below that, 128-column
+    // Column tiles of 256 (the down GEMM's) while they cover the CUs; below that, 128-column
     // tiles (one 32-row weight tile per wave, the same MFMA sequence per
     // column, so the same results), twice the workgroups. T = 2048: N = 2816
     // runs 352 narrow workgroups instead of 176 wide ones, 0.84-0.92 of the
