@@ -661,11 +661,13 @@ def test_default_stream_is_torchs_current_stream(tsg, ctx):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("m,n", [(1, 64), (17, 3072), (33, 3136), (48, 4096), (15, 4160), (31, 8256)])
+@pytest.mark.parametrize("m,n", [(1, 64), (9, 512), (18, 576), (17, 3072), (33, 3136), (48, 4096),
+                                 (15, 4160), (31, 8256)])
 @pytest.mark.parametrize("group,scheme", [(32, "sym"), (64, "affine")])
 def test_qmv_row_lengths_around_the_batches(tsg, ctx, m, n, group, scheme):
     """One batch of six chunks a lane covers n = 3072, one of eight n = 4096;
-    beyond, batches follow each other. Every row count gives the one-row
+    beyond, batches follow each other; n = 512 fills one chunk a lane, 576 two
+    lanes' second. Every row count gives the one-row
     result bit for bit, and that is DequantInt4GemvRef's within 1e-3."""
     configure(ctx, group, scheme)
     sym = scheme == "sym"

@@ -1365,9 +1365,9 @@ static_assert(64u * kSplitWaves == 32u * 16u, "one thread per pair of outputs");
 //  - one step: K = 2816, 9 rows x 4096 21.0 and 8.3, 32 rows 21.2 and 12.2, 64
 //    rows 23.4 and 12.6; K = 704, 256 x 1024 10.5 and 7.0. With K below 704 the
 //    split's fixed part is most of it: 32 rows x 2048 lose from K = 256 (affine
-//    g64 384: 5.4 and 6.0, 192: 5.2 and 4.9), affine 40 too (448: 5.7 and 6.1),
-//    24 and 96 rows gain. K = 512 loses nearly everywhere (32 x 8192 6.3 and
-//    8.4, 96 x 2688 7.8 and 8.4, 128 rows affine g32 9.0 and 9.5): rows an odd
+//    g64 384: 5.5 and 6.0, 192: 4.1 and 3.9), affine 40 x 4096 too (g64 448: 6.3
+//    and 6.7), 24 and 96 rows gain. K = 512 loses nearly everywhere (32 x 8192
+//    6.2 and 8.3, 96 x 2688 7.7 and 8.4, 128 rows affine g32 9.1 and 9.4): rows an odd
 //    multiple of 1 KB apart meet in the L1, as those of K = 2560 and 3584 do
 //    (64 x 4160, us a chunk: 0.59 at 2560, 0.50 at 2816, 0.49 at 3072), and
 //    there it is a short K besides.

@@ -13,7 +13,7 @@
 // cache holds, us before and now, group 32 sym: 704 x 2816 3.90 -> 3.26, 2816 x
 // 4096 6.12 -> 4.23, 4096 x 2816 3.95 -> 3.82; five rows of them 9.25 -> 5.98,
 // 15.95 -> 7.75, 7.23 -> 6.42; group 64 affine 2816 x 4096 6.35 -> 4.86, five
-// rows 17.5 -> 10.2, eight 68 -> 14.3.
+// rows 17.5 -> 9.1, eight 68 -> 12.4.
 #include "gemv_lane.hpp"
 
 namespace tsg {
@@ -23,21 +23,36 @@ constexpr uint32_t kMaxRows = 8;
 
 // compute_batch for T token rows, the rows' dot2 chains side by side (one
 // after the other, a wave waits for each dot2 of a 16-long chain: eight rows of
-// 8192 x 2816 12.1 us against 10.9, of 2816 x 4096 14.7 against 10.4). Each row takes compute_batch's steps.
+// 8192 x 2816 12.1 us against 10.9, of 2816 x 4096 14.7 against 10.4). Each row
+// takes compute_batch's steps.
+// Affine, several rows: the chunk sums are read ahead and the empty asm keeps
+// each row's value out of a branch on c < nchunks. Left alone, the compiler
+// makes that branch, a row and chunk at a time, and moves the row's dot2 chain
+// and its chunk sum's read behind it. Chunk slots that no lane has are passed
+// over instead (the branch's one use). us, one chain after the other with
+// batches of six, that branch, and now: five rows of 2816 x 4096 18.4, 10.3,
+// 9.1; eight of 8192 x 1024 8.0, 9.7, 7.3, of 8192 x 512 6.9, 8.7, 5.9. Sym
+// keeps its selects (five rows of 2816 x 4096 7.8; passing over slots 8.1),
+// and so does one row.
 template <int G, bool SYM, int KB, int T>
 __device__ __forceinline__ void compute_rows(const ChunkBatch<KB>& bt, uint32_t base, uint32_t j,
                                              uint32_t nchunks, const uint16_t* xs, uint32_t row_h,
                                              const float* xsum, float (&acc)[T]) {
+    constexpr bool kAffineRows = !SYM && T > 1;
     const h2_t bias = SYM ? h2_t{(_Float16)1032.0f, (_Float16)1032.0f}
                           : h2_t{(_Float16)1024.0f, (_Float16)1024.0f};
 #pragma unroll
     for (int i = 0; i < KB; ++i) {
+        if (kAffineRows && base + kGULanes * i >= nchunks) break;
         const uint32_t c = base + j + kGULanes * i;
         const uint32_t cc = min(c, nchunks - 1u);
         const uint32_t w[4] = {bt.w[i].x, bt.w[i].y, bt.w[i].z, bt.w[i].w};
-        float dot[T];
+        float dot[T], sums[T];
 #pragma unroll
-        for (int r = 0; r < T; ++r) dot[r] = 0.0f;
+        for (int r = 0; r < T; ++r) {
+            dot[r] = 0.0f;
+            sums[r] = kAffineRows ? xsum[r * nchunks + cc] : 0.0f;
+        }
 #pragma unroll
         for (int b = 0; b < 4; ++b) {
             h2_t q[4];
@@ -54,7 +69,8 @@ __device__ __forceinline__ void compute_rows(const ChunkBatch<KB>& bt, uint32_t 
 #pragma unroll
         for (int r = 0; r < T; ++r) {
             float v = __builtin_fmaf(s, dot[r], acc[r]);
-            if constexpr (!SYM) v = __builtin_fmaf(bi, xsum[r * nchunks + cc], v);
+            if constexpr (!SYM) v = __builtin_fmaf(bi, kAffineRows ? sums[r] : xsum[r * nchunks + cc], v);
+            if constexpr (kAffineRows) asm volatile("" : "+v"(v));
             acc[r] = c < nchunks ? v : acc[r];  // a chunk past the row end leaves acc as it is
         }
     }
@@ -139,8 +155,9 @@ __global__ __launch_bounds__(kQmvThreads) void qmv_kernel(const uint8_t* __restr
 // qmv_kernel does, and act = half(gelu(half(gate)) * half(up)) is gelu_mul's
 // (shared.hip). The halves are left in the caller's scratch too, as the
 // separate launches leave them (the three stores by one lane in their order:
-// the activation may share a buffer with either half). One launch for three, and one staging of x:
-// 2112 x 2816 in a 30-layer pass 3.9 + 3.9 + 2.0 us against 5.1.
+// the activation may share a buffer with either half). One launch for three,
+// and one staging of x: 2112 x 2816 in a 30-layer pass 3.9 + 3.9 + 2.0 us
+// against 5.1.
 template <int G, bool SYM, int WA, int KB>
 __global__ __launch_bounds__(kQmvThreads) void mlp_gate_up_kernel(
     const uint8_t* __restrict__ gate_w, const uint8_t* __restrict__ up_w,
