@@ -85,7 +85,7 @@ def test_prompt_router_equals_decode_router(tsg, ctx, t, ne, d):
     pes = dev(oracle.bf16_bits(rng.uniform(0.5, 1.5, ne).astype(np.float32)))
     moe = tsg.MoE(ctx)
     idx, wts = empty(t * 8, np.uint32), empty(t * 8)
-    for _ in range(2):  # the second call finds the row counters as the first left them
+    for _ in range(2):  # the second call finds the context's logits as the first left them
         idx.fill_(-1), wts.fill_(-1)
         tsg.PrefillRouter(moe).encode_gemma4_bf16(W, X, stride, es, pes, idx, wts, t, ne, d)
     gi = host(idx, np.uint32).reshape(t, 8)
@@ -97,6 +97,54 @@ def test_prompt_router_equals_decode_router(tsg, ctx, t, ne, d):
                                       one_i[8 * q:8 * q + 8], one_w[8 * q:8 * q + 8], ne, d)
     assert np.array_equal(gi[rows], host(one_i, np.uint32).reshape(-1, 8))
     assert np.array_equal(gw[rows], host(one_w, np.uint16).reshape(-1, 8))
+
+
+@pytest.mark.parametrize("t,ne,d", [(33, 128, 1544), (80, 256, 2816)])
+@pytest.mark.parametrize("kind", ["infinite", "subnormal", "overflow", "exact"])
+def test_prompt_router_keeps_the_order_at_the_ends_of_fp32(tsg, ctx, t, ne, d, kind):
+    """Where an MFMA could differ from the decode router's chain of fmas: rows
+    with infinite activations (one, two of a sign, two of both), logits that are
+    subnormal (their order is the only thing that ranks the experts), partial
+    sums that pass the largest number or cancel just below it, and integer logits
+    whose sums are exact only in order (2^24 and ones). Ids equal, weights equal
+    or both NaN."""
+    configure(ctx, 32, "sym")
+    rng = np.random.default_rng(t + d)
+    hidden = rng.normal(size=(t, d)).astype(np.float16)
+    w = rng.normal(0.0, d ** -0.5, (ne, d)).astype(np.float32)
+    es = rng.uniform(0.5, 1.5, d).astype(np.float32)
+    if kind == "infinite":
+        hidden[::3, 5] = np.inf
+        hidden[1::3, 64] = -np.inf
+        hidden[6::9, 700] = np.inf
+        hidden[9::9, 701] = -np.inf
+    elif kind == "subnormal":
+        es *= np.float32(2.0 ** -126)
+        w *= np.float32(2.0 ** -7)
+    elif kind == "overflow":
+        es *= np.float32(2.0 ** 121)
+        w *= np.float32(d ** 0.5 * 4.0)
+    else:
+        hidden = rng.choice([-1.0, 1.0], (t, d)).astype(np.float16)
+        w = rng.choice([1.0, 2.0 ** 24, -2.0 ** 24], (ne, d), p=[0.5, 0.25, 0.25]).astype(np.float32)
+        es = np.ones(d, np.float32)
+    W, X = dev(oracle.bf16_bits(w).ravel()), dev(hidden.view(np.uint16).ravel())
+    E = dev(oracle.bf16_bits(es))
+    pes = dev(oracle.bf16_bits(rng.uniform(0.5, 1.5, ne).astype(np.float32)))
+    moe = tsg.MoE(ctx)
+    idx, wts = empty(t * 8, np.uint32), empty(t * 8)
+    tsg.PrefillRouter(moe).encode_gemma4_bf16(W, X, d, E, pes, idx, wts, t, ne, d)
+    one_i, one_w = empty(t * 8, np.uint32), empty(t * 8)
+    for row in range(t):
+        moe.encode_router_gemma4_bf16(W, X[row * d:row * d + d], E, pes,
+                                      one_i[8 * row:8 * row + 8], one_w[8 * row:8 * row + 8], ne, d)
+    ids = host(one_i, np.uint32).reshape(t, 8)
+    got, want = host(wts, np.uint16).view(np.float16), host(one_w, np.uint16).view(np.float16)
+    assert np.array_equal(host(idx, np.uint32).reshape(t, 8), ids)
+    assert np.array_equal(got.view(np.uint16)[~np.isnan(want)], want.view(np.uint16)[~np.isnan(want)])
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    if kind in ("subnormal", "exact"):  # the case ranks, it does not tie
+        assert len(np.unique(ids)) > ne // 2 and not np.isnan(want).any()
 
 
 def _upload_layer(tsg, ctx, expert_parts, symmetric):
