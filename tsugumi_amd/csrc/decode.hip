@@ -856,8 +856,8 @@ __global__ __launch_bounds__(STAGE ? 64u * kStageWaves : 256u) void router_kerne
     const uint16_t* __restrict__ w, const uint16_t* __restrict__ hidden,
     const uint16_t* __restrict__ es, const uint16_t* __restrict__ pes,
     uint32_t* __restrict__ counters, uint32_t hidden_stride, uint32_t ne, uint32_t d,
-    uint32_t rows, float* __restrict__ logits, uint32_t* __restrict__ out_idx, uint16_t* __restrict__ out_w, uint32_t top_k,
-    RouterGroupOut grp) {
+    uint32_t rows, float* __restrict__ logits, uint32_t* __restrict__ out_idx,
+    uint16_t* __restrict__ out_w, uint32_t top_k, RouterGroupOut grp) {
     static_assert(!GROUP || (SELECT && STAGE), "the grouping follows a staged selection");
     static_assert(!STAGE || SELECT, "the staged form selects");
     extern __shared__ __align__(16) uint4 xrows[];  // STAGE: the block's rows, d / 8 units each

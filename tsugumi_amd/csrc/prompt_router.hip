@@ -12,10 +12,14 @@
 // chunk and the tree is added from the accumulators.
 //
 // What bounds it: the fp32 matrix rate. 2 T E d flops at 157 TFLOP/s are 9.4 us
-// for T = 2048, E = 128, d = 2816 and 27 us for T = 4096, E = 256, d = 2048;
-// both launches take 24.4 and 61.6 us there, 12.7 us for T = 67 and 13.3 for
-// T = 509. One wave an expert on vector fmas, each converting every row's
-// activations again, took 167, 617, 28 and 60 us.
+// for T = 2048, E = 128, d = 2816 and 27 us for T = 4096, E = 256, d = 2048.
+// Both launches, back to back in a HIP graph over router weights in turn, take
+// 25.1-25.7 and 63.0 us there, 13.0 for T = 67 and 14.0 for T = 509; of it the
+// selection 4.5, 5.1 and 3.9 us (kernel trace: 22.1 + 4.5, 62.7 + 5.1, 10.3 +
+// 3.9; in a prompt's layer, with other kernels between, 27.6 + 5.7 for T =
+// 2048). One wave an expert on vector fmas, each converting every row's
+// activations again, took 192 and 612 us, 29 for T = 64 and 44 for T = 300
+// (13.2 and 13.6 here).
 #include "router_select.hpp"
 #include <type_traits>
 
@@ -58,8 +62,9 @@ __device__ __forceinline__ void take_larger(uint32_t& key, uint32_t& inv) {
 // r. Lane l holds experts l + 16 j; 16 lanes a row keep every step inside the
 // DPP row, where a whole wave a row would take four times the rounds.
 template <int NJ>
-__device__ __forceinline__ void row16_top8(const float* __restrict__ logits, uint32_t ne, const uint16_t* __restrict__ gains,
-                                           uint32_t& id, uint16_t& weight) {
+__device__ __forceinline__ void row16_top8(const float* __restrict__ logits, uint32_t ne,
+                                           const uint16_t* __restrict__ gains, uint32_t& id,
+                                           uint16_t& weight) {
     const uint32_t l16 = threadIdx.x & 15u;
     uint32_t key[NJ];
 #pragma unroll
@@ -164,7 +169,7 @@ __device__ __forceinline__ float half_times(uint32_t x, uint32_t e) {
 // fp32 MFMAs and VALU instructions share their units here (each VALU
 // instruction between two MFMAs adds its own issue time, the first one twice
 // that), so the operands come out of LDS ready for use: only x * es is left to
-// compute. The last workgroup of a row tile to finish selects, four rows a wave.
+// compute. prompt_top8_kernel selects from the logits.
 template <int EA, int RB>
 __global__ __launch_bounds__(kPromptThreads) void prompt_router_kernel(
     const uint16_t* __restrict__ w, const uint16_t* __restrict__ hidden,

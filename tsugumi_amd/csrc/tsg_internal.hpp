@@ -104,9 +104,9 @@ constexpr uint32_t kMaxCounters = 12288;
 constexpr uint32_t kMaxGemmQueues = 8;                 // the fused GEMM's per-XCD queues
 constexpr uint32_t kGemmSchedBlocks = 65536;             // routed blocks the fused GEMM takes
 constexpr uint32_t kGemmSchedWords = 16u + kGemmSchedBlocks;
-// Words of ctx->counters used by the one-launch decode layer (below them, words
-// [0, kMaxPromptRows / 16) are the router's per-row-group completion
-// counters). Each area starts on its own 128-byte line.
+// Words of ctx->counters used by the one-launch decode layer (below them, word 0
+// is the one-row routers' completion counter). Each area starts on its own
+// 128-byte line.
 constexpr uint32_t kDecodeGroups = 8;      // one expert slot per group
 constexpr uint32_t kGroupMembers = 32;     // blocks per group
 constexpr uint32_t kDecodeBlocks = kDecodeGroups * kGroupMembers;
@@ -399,7 +399,8 @@ __device__ __forceinline__ uint4 pair_permute(uint4 v) {
 
 // The fp32 sum of each 32-element chunk of `rows` staged rows, in element
 // order, into sums[r * n/32 + c] (the affine scheme's bias term), from four
-// 16-byte reads a chunk. The staged rows must be visible to the block (the caller synchronises before).
+// 16-byte reads a chunk. The staged rows must be visible to the block (the
+// caller synchronises before).
 __device__ __forceinline__ void staged_chunk_sums(const uint16_t* dst, uint32_t dst_stride,
                                                   uint32_t rows, uint32_t n, float* sums) {
     const uint32_t cpr = n / 32u;
