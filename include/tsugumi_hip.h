@@ -604,11 +604,10 @@ tsg_status tsg_prefill_moe_down(tsg_moe* moe, tsg_stream stream, const tsg_layer
  * launch: exactly tsg_prefill_moe_gate_up followed by tsg_prefill_moe_down on
  * the same arguments (bit-identical act and route_partials), with the down
  * tiles of a block starting as soon as that block's gate/up tiles are done;
- * a device-counted list of few rows an expert runs as two launches of smaller
- * kernels instead, with the same bits: one whose capacity n_blocks is at most
- * the layer's experts + 16 (+ 6 under affine), d * f at most 2^21. The capacity
- * tsg_prefill_group_pairs_device asks for is that up to 16 * tile_rows pairs
- * (6 * tile_rows); entries to spare keep the one launch.
+ * a device-counted list of few rows an expert runs as the two launches, which
+ * are the faster there: one whose capacity n_blocks is at most the layer's
+ * experts + 32. The capacity tsg_prefill_group_pairs_device asks for is that up
+ * to 32 * tile_rows pairs; entries to spare keep the one launch.
  * The reference has no single call for the pair; a caller that issues the two
  * encodes back to back replaces them with this one. act must be 128-byte
  * aligned (TSG_ERR_ALIGNMENT); at most 65536 blocks. The schedule words live

@@ -524,7 +524,7 @@ def run_fused_vs_two_launches(tsg, ctx, layer, t, d, f, ne, s, act, seed, tile=2
     """tsg_prefill_moe_gate_up_down against tsg_prefill_moe_gate_up then
     tsg_prefill_moe_down on the same grouping: act and route partials equal
     bit for bit. A device list has 40 entries to spare: a tight one of few
-    pairs would take the few-rows kernels in place of the fused launch."""
+    pairs would run as two launches in place of the fused one."""
     k = 8
     rng = np.random.default_rng(seed)
     idx, w = wl.zipf_routing(rng, t, ne, k, s)
@@ -603,7 +603,7 @@ def test_grouped_gemm_skips_and_reports_expert_past_layer(tsg, ctx, gemma_layer,
     naming an expert past the layer is skipped by the grouped GEMM (two-launch
     and one-call forms) and tsg_ctx_synchronize reports it; the other blocks'
     rows are written as usual. The list is host-counted (0), or device-counted
-    with a capacity of the few-rows kernels (2) or of the wide ones (200)."""
+    with a capacity that the one call runs as two launches (2) or one (200)."""
     configure(ctx, 32, "sym")
     layer = gemma_layer[0]
     d, f, k, t = 2816, 704, 8, 4
@@ -635,13 +635,13 @@ def test_grouped_gemm_skips_and_reports_expert_past_layer(tsg, ctx, gemma_layer,
     ctx.synchronize()  # the error word was cleared
 
 
-@pytest.mark.parametrize("few_rows", [False, True])
-def test_fused_gate_up_down_zero_row_blocks(tsg, ctx, gemma_layer, few_rows):
+@pytest.mark.parametrize("device_list", [False, True])
+def test_fused_gate_up_down_zero_row_blocks(tsg, ctx, gemma_layer, device_list):
     """Routed blocks with no rows, between real ones, are no-ops in both
     forms: the fused launch (64 blocks, 1,088 items, so every workgroup takes
     several and meets zero-row items after others) equals the two launches
-    bit for bit and drains its schedule, twice in a row; so do the few-rows
-    kernels, which a device-counted list of that capacity takes."""
+    bit for bit and drains its schedule, twice in a row; so does the call with a
+    device-counted list of that capacity, which it runs as two launches."""
     configure(ctx, 32, "sym")
     layer = gemma_layer[0]
     d, f, k, t = 2816, 704, 8, 64
@@ -663,7 +663,7 @@ def test_fused_gate_up_down_zero_row_blocks(tsg, ctx, gemma_layer, few_rows):
     g.encode_down(layer, a2, P, B, 64, p2, k, d, f)
     want_a, want_p = host(a2, np.uint16), host(p2, np.uint16)
     assert np.all(np.isfinite(oracle.f16_to_float(want_p)))
-    count = dev(np.array([64], np.uint32)) if few_rows else None
+    count = dev(np.array([64], np.uint32)) if device_list else None
     for rep in range(2):
         a1, p1 = empty(t * k * f, fill=NAN16), empty(t * k * d, fill=NAN16)
         g.encode_gate_up_down(layer, hidden, d, P, B, 64, a1, p1, k, d, f, n_blocks_device=count)
@@ -675,9 +675,9 @@ def test_fused_gate_up_down_zero_row_blocks(tsg, ctx, gemma_layer, few_rows):
 @pytest.mark.parametrize("capacity", [1, 200])
 def test_fused_gate_up_down_empty_device_list(tsg, ctx, gemma_layer, capacity):
     """A device count of zero (no routed block) runs the fused launch (capacity
-    200; the few-rows kernels at 1) to its end without work, writes nothing and
-    reports nothing; the next launch on the same context still runs a real
-    list (the schedule was left reset)."""
+    200; two launches at 1) to its end without work, writes nothing and reports
+    nothing; the next launch on the same context still runs a real list (the
+    schedule was left reset)."""
     configure(ctx, 32, "sym")
     layer = gemma_layer[0]
     d, f, k, t = 2816, 704, 8, 4

@@ -492,166 +492,6 @@ __device__ __forceinline__ void gemm_kloop(const GemmLane<NT>& L, uint8_t* smem,
     }
 }
 
-// ---- the K loop of the thin kernels (passes of at most kThinRows rows)
-//
-// A chunk's activations (NT slices) and weights share an LDS stage; the loop
-// over chunks is rolled, with the stage as a run-time offset, kStages - 1
-// chunks ahead (gate/up: sym 4 of one slice and 3 of two, affine 3 and 2; down:
-// sym 3 and 2, affine 2 and 1). One barrier a chunk: it publishes chunk c and
-// frees chunk c - 1's stage. Every accumulator sees gemm_kloop's MFMA sequence,
-// so the results are the same.
-// Group parameters: a dword a row and chunk is a load of 64 lines for 4 bytes
-// of each, and where K is long those lines and the weights' outgrow the L2
-// before their next dword is read. Gate/up (K = d) therefore takes the wide
-// kernels' 16-byte windows of four chunks, in three buffers past the stages,
-// with two workgroups per CU; down (K = f, whose parameter rows lie a few to a
-// line) the chunk's dword in its stage, with three.
-constexpr uint32_t kThinRows = 64u;
-__host__ __device__ constexpr uint32_t thin_per_cu(int mode) { return mode == 0 ? 2u : 3u; }
-template <bool SYM, int NT, int MODE>
-struct ThinLds {
-    static constexpr bool kWindows = MODE == 0;
-    static constexpr uint32_t kBytes = MODE == 0 ? 81920u : 53248u;
-    static constexpr uint32_t kB = NT * 4096u;                  // after the activations
-    static constexpr uint32_t kS = kB + kGemmBStage;            // no windows: 64 rows x 4 bytes a wave
-    static constexpr uint32_t kZ = kS + kGemmWaves * 256u;
-    static constexpr uint32_t kStage = kWindows ? kS : kZ + (SYM ? 0u : kGemmWaves * 256u);
-    static constexpr uint32_t kBufs = 3u;                       // scale windows, then bias windows
-    static constexpr uint32_t kWin = kWindows ? kBufs * kGemmSBuf * (SYM ? 1u : 2u) : 0u;
-    static constexpr uint32_t kStages = (kBytes - kWin) / kStage;
-    static constexpr uint32_t kW = kStages * kStage;            // where the windows start
-    static_assert(kStage % 128u == 0 && kStages >= 2u, "ring");
-    static_assert(kBytes * thin_per_cu(MODE) <= 160u * 1024u, "workgroups per CU");
-    static_assert(GemmLds<kThinRows>::kEpi <= kBytes, "epilogue");
-    // chunk c reads its window after its loads are issued: window V last in
-    // chunk 4 V + 3, and the first piece of window V + kBufs goes out in chunk
-    // 4 (V + kBufs) - 3 - (kStages - 1)
-    static_assert(!kWindows || 4u * kBufs > kStages + 5u, "a window is read before it is overwritten");
-};
-
-// Piece q of window V (window_piece's load) into the buffer at `dst`.
-template <int G, bool SYM, int NT, int MODE>
-__device__ __forceinline__ void thin_window(const GemmLane<NT>& L, uint8_t* dst, uint32_t q, uint32_t V) {
-    using T = ThinLds<SYM, NT, MODE>;
-    const uint32_t row = (q & 1u) * L.s_q1, d4 = 4u * (threadIdx.x & 3u);
-    const uint32_t s = (q >= 2u ? L.s_ld[1] : L.s_ld[0]) + row, z = (q >= 2u ? L.z_ld[1] : L.z_ld[0]) + row;
-    uint8_t* to = dst + L.wave * kGemmSWave + q * 256u;
-    lds_buf4(L.sbuf, G == 32 ? s + 16u * V : ((s + 8u * V) & ~3u) + d4, 0u, to);
-    if constexpr (!SYM)
-        lds_buf4(L.zbuf, G == 32 ? z + 16u * V : ((z + 8u * V) & ~3u) + d4, 0u, to + T::kBufs * kGemmSBuf);
-}
-
-template <int G, bool SYM, int NT, int MODE>
-__device__ __forceinline__ void thin_issue(const GemmLane<NT>& L, uint8_t* smem, uint8_t* stage, uint32_t c) {
-    using T = ThinLds<SYM, NT, MODE>;
-#pragma unroll
-    for (int i = 0; i < NT; ++i)
-        lds_buf16(L.abuf, L.a_off[i], c * (kGemmKC * 2u), stage + L.wave * 1024u + (uint32_t)i * 4096u);
-    uint8_t* b = stage + T::kB + L.wave * kGemmBWave;
-    lds_buf16(L.wbuf, L.w_off[0], c * (kGemmKC / 2u), b);
-    lds_buf16(L.wbuf, L.w_off[1], c * (kGemmKC / 2u), b + kGemmBTile);
-    if constexpr (T::kWindows) {
-        const uint32_t V = (c + 3u) >> 2;
-        thin_window<G, SYM, NT, MODE>(L, smem + T::kW + V % T::kBufs * kGemmSBuf, (c + 3u) & 3u, V);
-    } else {
-        // lane l brings the dword with the chunk's group(s) of its row: row
-        // l % 32 of tile l / 32
-        const bool t1 = (threadIdx.x & 32u) != 0u;
-        const uint32_t s = t1 ? L.s_own[1] : L.s_own[0], z = t1 ? L.z_own[1] : L.z_own[0];
-        const uint32_t at = c * (G == 32 ? 4u : 2u);
-        lds_buf4(L.sbuf, G == 32 ? s + at : (s + at) & ~3u, 0u, stage + T::kS + L.wave * 256u);
-        if constexpr (!SYM)
-            lds_buf4(L.zbuf, G == 32 ? z + at : (z + at) & ~3u, 0u, stage + T::kZ + L.wave * 256u);
-    }
-}
-
-// a_rd, b_rd: the lane's read addresses of step 0's activations (slice 0) and
-// of its weights in stage 0; tile: the weight tile of slot 0 (HALF: 1 on the
-// waves that run the up rows).
-template <int G, bool SYM, int NT, bool HALF, int MODE>
-__device__ __forceinline__ void thin_kloop(const GemmLane<NT>& L, uint8_t* smem, uint32_t a_rd,
-                                           uint32_t b_rd, uint32_t tile, f16v_t (&acc)[NT][2]) {
-    using T = ThinLds<SYM, NT, MODE>;
-    constexpr uint32_t kLoads = (uint32_t)NT + (SYM ? 3u : 4u);
-    const uint32_t last = L.nchunks - 1u;
-    if constexpr (T::kWindows) {
-#pragma unroll
-        for (uint32_t q = 0; q < 3u; ++q) thin_window<G, SYM, NT, MODE>(L, smem + T::kW, q, 0u);
-    }
-    // chunks past the last repeat it: every chunk issues the same loads
-#pragma unroll
-    for (uint32_t q = 0; q < T::kStages - 1u; ++q)
-        thin_issue<G, SYM, NT, MODE>(L, smem, smem + q * T::kStage, q < last ? q : last);
-    const uint32_t m = threadIdx.x & 31u, h = (threadIdx.x >> 5) & 1u;
-    // windows: the lane's row's 16 bytes in buffer 0; G = 32, half h reads group
-    // 2 c + h, the second half of the chunk's dword; G = 64, the groups of a row
-    // that starts off a dword lie one half word on
-    const uint32_t s_rd = lds_addr(smem) + (T::kWindows
-                              ? T::kW + L.wave * kGemmSWave + (32u * tile + m) * 16u
-                              : T::kS + L.wave * 256u + (32u * tile + m) * 4u);
-    const uint32_t sw0 = s_rd + (G == 32 ? 2u * h : L.s_own[0] & 2u);
-    const uint32_t sw1 = s_rd + 512u + (G == 32 ? 2u * h : L.s_own[1] & 2u);
-    const uint32_t zw0 = s_rd + T::kBufs * kGemmSBuf + (G == 32 ? 2u * h : L.z_own[0] & 2u);
-    const uint32_t zw1 = s_rd + T::kBufs * kGemmSBuf + 512u + (G == 32 ? 2u * h : L.z_own[1] & 2u);
-    uint32_t win = 0u;  // chunk c's buffer and its groups there
-    uint32_t read = 0u, write = (T::kStages - 1u) * T::kStage;  // stages of chunk c and the one issued
-#pragma unroll 1
-    for (uint32_t c = 0; c < L.nchunks; ++c) {
-        wait_vmcnt<(T::kStages - 2u) * kLoads>();
-        block_barrier();
-        const uint32_t ahead = c + T::kStages - 1u;
-        thin_issue<G, SYM, NT, MODE>(L, smem, smem + write, ahead < last ? ahead : last);
-        u32x4_t af[2][NT], bw0, bw1;
-        const uint32_t a = a_rd + read, b = b_rd + read;
-        lds_read_act<NT, 0u>(af[0], a);
-        bw0 = lds_read16<0>(b);
-        bw1 = HALF ? bw0 : lds_read16<kGemmBTile>(b);
-        uint32_t s0, s1, z0 = 0u, z1 = 0u;
-        if constexpr (T::kWindows) {
-            s0 = lds_read_u16(sw0 + win);
-            s1 = HALF ? s0 : lds_read_u16(sw1 + win);
-            if constexpr (!SYM) {
-                z0 = lds_read_u16(zw0 + win);
-                z1 = HALF ? z0 : lds_read_u16(zw1 + win);
-            }
-            constexpr uint32_t kStep = G == 32 ? 4u : 2u;
-            win += (c & 3u) != 3u ? kStep : kGemmSBuf - 3u * kStep;
-            if (win == T::kBufs * kGemmSBuf) win = 0u;
-        } else {
-            // G = 32: half h takes the dword's group 2 c + h; G = 64: the half
-            // that the row's alignment puts the group in
-            const uint32_t sh0 = G == 32 ? 2u * h : (L.s_own[0] + 2u * c) & 2u;
-            const uint32_t sh1 = G == 32 ? 2u * h : (L.s_own[1] + 2u * c) & 2u;
-            s0 = lds_read_u16(s_rd + read + sh0);
-            s1 = HALF ? s0 : lds_read_u16(s_rd + read + 128u + sh1);
-            if constexpr (!SYM) {
-                const uint32_t zh0 = G == 32 ? 2u * h : (L.z_own[0] + 2u * c) & 2u;
-                const uint32_t zh1 = G == 32 ? 2u * h : (L.z_own[1] + 2u * c) & 2u;
-                z0 = lds_read_u16(s_rd + read + (T::kZ - T::kS) + zh0);
-                z1 = HALF ? z0 : lds_read_u16(s_rd + read + (T::kZ - T::kS) + 128u + zh1);
-            }
-        }
-        lds_wait<NT>(af[0], bw0, bw1, s0, s1, z0, z1);
-        const GroupScale g0 = group_scale<SYM>((uint16_t)s0, (uint16_t)z0);
-        const GroupScale g1 = group_scale<SYM>((uint16_t)s1, (uint16_t)z1);
-#pragma unroll
-        for (int st = 0; st < 4; ++st) {
-            if (st < 3) lds_read_act<NT, 0u>(af[(st + 1) & 1], step_addr(a, (uint32_t)(st + 1)));
-            const h8v_t w0 = dequant8<SYM>(bw0[st], g0), w1 = HALF ? w0 : dequant8<SYM>(bw1[st], g1);
-#pragma unroll
-            for (int i = 0; i < NT; ++i) {
-                const h8v_t x = __builtin_bit_cast(h8v_t, af[st & 1][i]);
-                acc[i][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x, w0, acc[i][0], 0, 0, 0);
-                if constexpr (!HALF)
-                    acc[i][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x, w1, acc[i][1], 0, 0, 0);
-            }
-            if (st < 3) lds_wait<NT>(af[(st + 1) & 1]);
-        }
-        read = read == (T::kStages - 1u) * T::kStage ? 0u : read + T::kStage;
-        write = write == (T::kStages - 1u) * T::kStage ? 0u : write + T::kStage;
-    }
-}
-
 // MODE 0: gate/up + activation; MODE 1: down + scatter; MODE 2: dense
 // projection y[t, n] (the down sub-tensor's geometry, rows taken in order).
 // HALF, dense GEMM: a 128-column tile, wave w the 32 weight rows 32 w .. of
@@ -672,12 +512,12 @@ __host__ __device__ constexpr uint32_t gemm_rows() { return MODE == 2 ? kDenseRo
 template <bool SYM>
 __host__ __device__ constexpr uint32_t next_word() { return GemmLds<kGemmRows>::kWord; }
 
-template <int G, bool SYM, int ACT, int MODE, int NT, bool HALF, bool THIN = false>
+template <int G, bool SYM, int ACT, int MODE, int NT, bool HALF>
 __device__ __forceinline__ void gemm_block(const GemmArgs& args, const tsg_routed_block& blk,
                                            uint32_t rows, uint32_t tile, uint8_t* smem,
                                            bool post, uint32_t next) {
     static_assert(!HALF || MODE != 1, "the down GEMM has no half tiles");
-    constexpr uint32_t R = THIN ? kThinRows : gemm_rows<MODE>();
+    constexpr uint32_t R = gemm_rows<MODE>();
     using Y = GemmLds<R>;
     static_assert(NT >= 1 && (uint32_t)NT <= Y::kSlices, "slices per pass");
     const uint32_t lane = threadIdx.x & 63u, h = lane >> 5, m = lane & 31u;
@@ -789,12 +629,7 @@ __device__ __forceinline__ void gemm_block(const GemmArgs& args, const tsg_route
         const tsg_token_expert_pair pr = args.pairs[blk.pair_start + threadIdx.x];
         row_dst = (pr.token * args.top_k + pr.rank) * args.d;
     }
-    if constexpr (THIN) {
-        const uint32_t up = MODE == 0 && HALF && L.wave >= 2u ? 1u : 0u;
-        thin_kloop<G, SYM, NT, HALF, MODE>(L, smem, L.a_rd, L.b_rd - Y::kBBase + NT * 4096u, up, acc);
-    } else {
-        gemm_kloop<R, G, SYM, NT, HALF>(L, smem, acc);
-    }
+    gemm_kloop<R, G, SYM, NT, HALF>(L, smem, acc);
     wait_vmcnt<0>();  // no LDS write may land after this point
 
     // Output: the block's tile goes through LDS (idle now) so
@@ -1023,50 +858,6 @@ __device__ __forceinline__ void gemm_item(const GemmArgs& args, const tsg_routed
     }
 }
 
-// The routed GEMMs of a call whose experts have few rows each, in passes of
-// kThinRows rows. Such a call is bound by latency: a weight is dequantised for
-// one or two MFMAs, so a chunk is barrier, LDS reads, dequantisation and MFMAs
-// in turn (0.5 us alone); deeper rings and, in down, three workgroups per CU
-// (the wide kernels' accumulators and rings allow two) hide more of it. Gate/up
-// and down of 67 tokens, 8 of 128 experts, 2816 x 704, sym g32, four layers in
-// turn, fused launch and here: logits with half their variance in common (67
-// experts) 131 and 93 us, with none (126 experts) 158 and 158; 9 tokens 94 and
-// 54, 125 and 96. With a dword of scales a row and chunk in gate/up too and
-// three workgroups per CU they were 104, 182, 56 and 105, and affine g32, which
-// reads twice the parameters, 134 and 274 for 67 tokens (107 and 192 here, 148
-// and 199 fused). Grid: x = items as in moe_gemm_kernel, y = the passes side
-// by side.
-template <int G, bool SYM, int ACT, int MODE>
-__global__ __launch_bounds__(kGemmThreads, thin_per_cu(MODE)) void moe_gemm_thin_kernel(GemmArgs args) {
-    extern __shared__ __align__(16) uint8_t smem[];  // ThinLds::kBytes
-    const uint32_t nb = args.n_blocks_device ? min(*args.n_blocks_device, args.n_blocks) : args.n_blocks;
-    if (blockIdx.x >= nb * args.ntiles) return;
-    uint32_t yb, tile;
-    gemm_work_item(args, nb, blockIdx.x, reinterpret_cast<uint32_t*>(smem), true, yb, tile);
-    const tsg_routed_block blk = args.blocks[yb];
-    // a block list written on the device is not checked on the host: an
-    // expert past the layer is skipped (its weights would lie outside it)
-    if (blk.local_slot >= args.num_experts) {
-        if (blk.row_count != 0 && threadIdx.x == 0) atomicOr(args.error, kErrGemmBlock);
-        return;
-    }
-    const bool half = MODE == 0 && args.f - tile * 128u <= 64u;
-    for (uint32_t r0 = blockIdx.y * kThinRows; r0 < blk.row_count; r0 += gridDim.y * kThinRows) {
-        if (r0 != blockIdx.y * kThinRows) lds_barrier();  // every wave is done with the previous pass's LDS
-        tsg_routed_block sub = blk;
-        sub.pair_start += r0;
-        sub.local_row += r0;
-        const uint32_t rows = blk.row_count - r0 < kThinRows ? blk.row_count - r0 : kThinRows;
-        if (rows > 32u) {
-            if (half) gemm_block<G, SYM, ACT, MODE, 2, MODE == 0, true>(args, sub, rows, tile, smem, false, 0u);
-            else gemm_block<G, SYM, ACT, MODE, 2, false, true>(args, sub, rows, tile, smem, false, 0u);
-        } else {
-            if (half) gemm_block<G, SYM, ACT, MODE, 1, MODE == 0, true>(args, sub, rows, tile, smem, false, 0u);
-            else gemm_block<G, SYM, ACT, MODE, 1, false, true>(args, sub, rows, tile, smem, false, 0u);
-        }
-    }
-}
-
 // 1-D grid of ntiles x (routed block capacity) workgroups; those past the
 // live count exit at once. Two workgroups per CU.
 template <int G, bool SYM, int ACT, int MODE>
@@ -1194,53 +985,12 @@ __global__ __launch_bounds__(kGemmThreads, 2) void moe_gemm_fused_kernel(GemmArg
 
 // ------------------------------------------------------------- launchers
 
-// Whether a device-written work list goes to the thin kernels. The host knows
-// of it only its capacity: of tsg_prefill_group_pairs_device's ceil(pairs /
-// tile_rows) + E entries, those past E count the pairs. 16 are 2048 pairs in
-// blocks of 128 rows, 4096 of 256, 1024 of 64. Fused launch and thin kernels,
-// us, 2816 x 704 of 128 experts, sym g32, logits with half their variance in
-// common and (in brackets) with none, the routing that reads most experts:
-// 2048 pairs 189 and 144 (159 and 155), 3072 196 and 169 (166 and 167), 4096
-// 199 and 181 (178 and 179), in blocks of 256 rows 280 and 210 (178 and 177);
-// 256 experts of 2048 x 512 131 and 102 (155 and 151) at 2048, in blocks of 256
-// 247 and 144 (158 and 155) at 4096. Few experts gain too (8 experts, 2048
-// pairs: 87 and 59). The worst met is 536 pairs evenly over 256 experts of 2048
-// x 512, 132 and 137. Affine lists stop at 6, 768 pairs of 128 rows (g64 150 and 104, 170
-// and 171 in brackets; g32 172 and 122, 201 and 197): at 2048 they would gain
-// too (189 and 150, 171 and 165) and are left as they were. Wider experts: 40
-// tokens over 64 experts of 2048 x 1024 are 108 and 71 (109 and 87), affine g32
-// 111 and 78; of 4096 x 1536 209 and 180 (234 and 229), affine 252 and 249 (302
-// and 307) and, 96 tokens, 285 and 313, so d * f stays at 2^21 (2816 x 704 is
-// 1.98 M). A list with spare capacity goes to the wide kernels, with the same
-// results.
-template <bool SYM>
-inline bool few_rows(const GemmArgs& a, uint32_t max_blocks) {
-    return a.n_blocks_device && max_blocks <= (uint64_t)a.num_experts + (SYM ? 16u : 6u) &&
-           (uint64_t)a.d * a.f <= 1u << 21;
-}
-
-template <int G, bool SYM, int MODE>
-tsg_status launch_thin(const tsg_moe* moe, hipStream_t s, const GemmArgs& args, uint32_t max_blocks) {
-    auto kern = moe->activation == TSG_ACT_SILU ? moe_gemm_thin_kernel<G, SYM, TSG_ACT_SILU, MODE>
-                                                : moe_gemm_thin_kernel<G, SYM, TSG_ACT_GELU_TANH, MODE>;
-    // the passes of a block of 128 rows run side by side; those of wider blocks
-    // (256 rows: four) two by two
-    const dim3 grid(args.ntiles * max_blocks, 2u);
-    constexpr uint32_t lds = ThinLds<SYM, 1, MODE>::kBytes;
-    if (lds > 64u * 1024u)
-        TSG_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(kern, grid, dim3(kGemmThreads), lds, s, args);
-    return check_launch(MODE == 0 ? "moe_gemm thin gate/up" : "moe_gemm thin down");
-}
-
 template <int G, bool SYM, int MODE>
 tsg_status launch_gemm(const tsg_moe* moe, hipStream_t s, const GemmArgs& a, uint32_t max_blocks) {
     GemmArgs args = a;
     args.ntiles = MODE == 0 ? (a.f + 127u) / 128u : (a.d + 255u) / 256u;  // 4 waves x 32 / 64 rows
     TSG_REQUIRE((uint64_t)args.ntiles * max_blocks <= 0x7FFFFFFFu, TSG_ERR_INVALID_ARGUMENT,
                 "moe_gemm: %u routed blocks x %u tiles exceed the grid", max_blocks, args.ntiles);
-    if (MODE != 2 && few_rows<SYM>(args, max_blocks)) return launch_thin<G, SYM, MODE>(moe, s, args, max_blocks);
     const dim3 grid(args.ntiles * max_blocks);
     auto kern = moe->activation == TSG_ACT_SILU ? moe_gemm_kernel<G, SYM, TSG_ACT_SILU, MODE>
                                                 : moe_gemm_kernel<G, SYM, TSG_ACT_GELU_TANH, MODE>;
@@ -1252,10 +1002,31 @@ tsg_status launch_gemm(const tsg_moe* moe, hipStream_t s, const GemmArgs& a, uin
     return check_launch(MODE == 0 ? "moe_gemm gate/up" : "moe_gemm down");
 }
 
+// Whether the pair runs as two launches instead of the persistent one, which
+// pays where down's items fill the tail of gate/up's. With few rows an expert
+// the items are short and many of them start by waiting (for the next index,
+// for their block's gate/up tiles). The host knows of a device-written list only
+// its capacity; of tsg_prefill_group_pairs_device's ceil(pairs / tile_rows) + E
+// entries, those past E count the pairs: 32 are 4096 pairs in blocks of 128
+// rows, 8192 of 256, 2048 of 64. Persistent and two launches, us, four layers in
+// turn, sym g32 of 128 experts of 2816 x 704, logits with half their variance in
+// common and (in brackets) none, the routing that reads most experts: 9 tokens
+// 100 and 56 (130 and 91), 67 146 and 97 (159 and 145), 256 194 and 136 (162 and
+// 150), 512 202 and 169 (180 and 173), in blocks of 256 0.58 (0.97) of the time,
+// of 64 0.98 (0.96); affine g32 of 67 tokens 154 and 106 (197 and 185). 1024
+// tokens are 225 and 209 (206 and 204), 2048 306 and 315 (302 and 313). Over
+// eight layer shapes (8 to 256 experts, 768 x 256 to 4096 x 1536) no list up to
+// 4096 pairs was slower by more than 4 % (536 pairs evenly over 256 experts of
+// 2048 x 512: 132 and 137). A list with spare capacity keeps the one launch, with
+// the same results.
+inline bool few_rows(const GemmArgs& a, uint32_t max_blocks) {
+    return a.n_blocks_device && max_blocks <= (uint64_t)a.num_experts + 32u;
+}
+
 template <int G, bool SYM>
 tsg_status launch_fused(const tsg_moe* moe, hipStream_t s, GemmArgs gu, GemmArgs dn,
                         uint32_t max_blocks) {
-    if (few_rows<SYM>(gu, max_blocks)) {
+    if (few_rows(gu, max_blocks)) {
         const tsg_status st = launch_gemm<G, SYM, 0>(moe, s, gu, max_blocks);
         return st ? st : launch_gemm<G, SYM, 1>(moe, s, dn, max_blocks);
     }
