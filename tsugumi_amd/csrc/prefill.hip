@@ -189,8 +189,8 @@ __global__ __launch_bounds__(256) void group_scatter_kernel(
 // and here: 9 tokens of top-8 over 128 experts 8.2 and 4.1, 128 tokens 8.5 and
 // 4.3, 256 8.4 and 5.2. One CU's stores of the pairs grow with their number
 // (400 tokens 8.3 and 7.0, 512 8.3 and 7.4), so the line is at 2048 pairs,
-// below which a whole prompt layer gains what the grouping does (9 tokens 79.6
-// -> 75.2, 128 tokens 167.4 -> 163.1) and above which it did so within noise.
+// below which a whole prompt layer gains what the grouping does (9 tokens 4.4,
+// 128 tokens 4.3) and above which it did so within noise.
 constexpr uint32_t kSmallPairs = 2048u;
 constexpr uint32_t kSmallThreads = 1024u, kSmallWaves = kSmallThreads / 64u;
 constexpr uint32_t kSmallSteps = kSmallPairs / kSmallThreads;
